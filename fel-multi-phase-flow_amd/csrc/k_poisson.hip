@@ -673,7 +673,10 @@ void tdma1_t(const Dims d, const double* div, double* phir_r, double* phir_i) {
   if constexpr (is_f32<T>)
     warm = refine_steps() > 0 && rec.coef && rec.dp_host && rec.ni == d.ni && rec.nj == d.nj &&
            rec.nk == d.nk && content_version(div, d.n3) != 0 &&
-           content_version(rec.dp_host, d.n3) != 0;
+           content_version(rec.dp_host, d.n3) != 0 &&
+           // the last solve's array may be gone and its address another's
+           // (any FP64 array is a starting guess)
+           elem_size(rec.dp_host) == (int)sizeof(double);
   Call c("solp_fft_tdma1_");
   const PT<T>* dv = c.in_t<PT<T>>(div, d.n3, "div");
   T* pr = c.out_t<T>(phir_r, nm, "phir_r");

@@ -117,6 +117,65 @@ def test_fp32_pressure_correction(fp32_modes, tol, bar):
         _set_refinement(3, 1e-7)
 
 
+def test_warm_start_after_the_correction_array_is_gone():
+    """The address of the last FP32 solve's correction may since hold a
+    flow-class array of the same size: the next solve starts cold instead of
+    reading it as FP64."""
+    g = H.Grid(16, 8, 16)
+    lib = H.gpu()
+    lib.felgpu_set_precision_(ctypes.byref(ctypes.c_int(32)))
+    reg = []
+
+    def register(a, fp64, upload=1):
+        fn = lib.felgpu_register_fp64_ if fp64 else lib.felgpu_register_
+        fn(ctypes.c_void_p(a.ctypes.data), ctypes.byref(ctypes.c_int64(a.nbytes)),
+           ctypes.byref(ctypes.c_int(upload)))
+        reg.append(a)
+
+    def drop(a):
+        lib.felgpu_unregister_(ctypes.c_void_p(a.ctypes.data))
+        reg[:] = [x for x in reg if x is not a]
+
+    try:
+        r = np.random.default_rng(55)
+        div, div2, old, new = (g.zeros() for _ in range(4))
+        g.interior(div)[...] = r.standard_normal((g.nk, g.nj, g.ni))
+        g.interior(div)[...] -= g.interior(div).mean()
+        div2[...] = div
+        modes = [np.zeros(g.ni * g.nj * g.nk) for _ in range(2)]
+        head = [I(g.ni), I(g.nj), I(g.nk)]
+        pc = [np.zeros(g.nj + 6) for _ in range(7)]
+        fft = [np.zeros(g.nj + 6) for _ in range(3)]
+        H.call_gpu("cal_coef_prs", I(g.nj), D(1.0), D(1.0), D(1.0), D(1.0), *pc)
+        H.call_gpu("cal_coef_solp_fft", I(g.nj), pc[2], pc[3], *fft)
+        sv = np.array([g.ni, g.nj, g.nk], dtype=np.int32)
+        wk = [np.zeros(64) for _ in range(3)]
+
+        def solve(rhs, dp):
+            H.call_gpu("solp_fft_tdma1", *head, wk[0], rhs, *modes)
+            H.call_gpu("solp_fft_tdma2", I(0), I(1), sv, D(1.0), D(1.0), D(1.0), *fft, *wk, *modes)
+            H.call_gpu("solp_fft_tdma3", *head, wk[0], *modes, dp)
+            lib.felgpu_download_(ctypes.c_void_p(dp.ctypes.data))
+            return g.interior(dp).copy()
+
+        for a in (div, old):
+            register(a, True)
+        for a in modes:
+            register(a, False, 0)
+        first = solve(div, old)
+        drop(old)
+        old[...] = r.standard_normal(g.shape)
+        register(old, False)  # the same address, now a flow-class array
+        register(div2, True)
+        register(new, True)
+        second = solve(div2, new)
+        assert np.linalg.norm(first - second) <= 1e-5 * np.linalg.norm(first)
+    finally:
+        for a in list(reg):
+            drop(a)
+        lib.felgpu_set_precision_(ctypes.byref(ctypes.c_int(64)))
+
+
 def test_fp32_precision_is_per_array_class():
     """Flow arrays registered with felgpu_register_ are FP32, arrays
     registered with felgpu_register_fp64_ stay FP64; a kernel asked to read
