@@ -1,0 +1,46 @@
+"""The launch shapes that depend on the grid: chunk lengths of the marching
+kernels, tile edges and remainders, each against the oracle on the sizes where
+a shape changes."""
+import numpy as np
+import pytest
+
+import felharness as H
+from felharness import D, I, Grid
+from test_gpu_kernels import check, grad, run_both
+
+pytestmark = pytest.mark.gpu
+
+
+# (64 x 4 blocks; one plane per thread up to 8: 4^3 and the odd grids march one
+# plane, 130 x 40 x 40 two, 200 x 100 x 70 eight)
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (63, 5, 9), (66, 7, 18), (130, 40, 40),
+                                      (200, 100, 70)])
+@pytest.mark.parametrize("flat", [False, True], ids=["interface", "flat"])
+def test_mthinc_flux_and_truncation_shapes(ni, nj, nk, flat):
+    """solphi_mthinc1 with and without interface cells, and the truncation
+    pass of solphi_mthinc3.  Bars: the fluxes' Gauss sums differ from the
+    oracle's by the rounding of an 8-term sum and of the device's exp (1e-13
+    of the largest flux); phin by the mass offset's sum order."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 16, 1 / 16)
+    r = np.random.default_rng(ni + nj + nk)
+    phi = np.full(g.shape, 0.75) if flat else H.smooth_phi(g, r)
+    gx, gy, gz = grad(g, phi)
+    u, v, w = (H.random_vel(g, r, 0.5) for _ in range(3))
+    u[3, 3, 3] = v[4, 4, 4] = w[5, 5, 5] = 0.0
+    head = [I(g.ni), I(g.nj), I(g.nk), D(1 / g.dx), D(1 / g.dy), D(1 / g.dz)]
+    old = [r.standard_normal(g.shape) for _ in range(3)]
+
+    def flux():
+        return head + [D(0.01), D(1.0), phi.copy(), gx.copy(), gy.copy(), gz.copy(), u.copy(),
+                       v.copy(), w.copy()] + [x.copy() for x in old]
+    check(*run_both("solphi_mthinc1", flux), rtol=1e-13)
+    phin = np.clip(phi + 0.01 * r.standard_normal(g.shape), -0.05, 1.05)
+
+    def trunc():
+        return [I(0)] + head + [D(1.0), gx.copy(), gy.copy(), gz.copy(), phi.copy(), phin.copy()]
+    a, b = run_both("solphi_mthinc3", trunc)
+    # the offset's two sums of n terms are taken in another order: each is off
+    # by at most n eps times itself; phin moves by offset p^2 (1-p) <= 4/27 offset
+    p = np.clip(g.interior(phin), 0.0, 1.0)
+    bar = 4 / 27 * 2 * p.size * 1.2e-16 * p.sum() / (p * p * (1 - p)).sum() + 1e-15
+    assert np.max(np.abs(a[-1] - b[-1])) <= bar
