@@ -29,7 +29,7 @@ void grad_p2uvw(const Dims d, int ID, double dxinv, const double* dyt_dev, doubl
 }
 
 // srcs/calrn.f:23-87.  One thread per target column (ii,jj), marching over
-// a chunk of kk planes: the four source values of plane kk are kept for the
+// a chunk of up to kRnChunk planes kk: the four source values of plane kk are kept for the
 // next plane, so each plane is loaded once per array instead of twice, and
 // the 8-term sums keep the reference's order (plane kk-kp first).  Targets
 // outside the shifted loop range keep the cleared value 0.
@@ -40,14 +40,14 @@ __global__ void __launch_bounds__(256) calrn_kernel(Dims d, T verysmall, int ip,
                                                     const T* __restrict__ px,
                                                     const T* __restrict__ py,
                                                     const T* __restrict__ pz, T* __restrict__ rn,
-                                                    int gx, int gy, int ntiles) {
+                                                    int gx, int gy, int ntiles, int kc) {
   const int L = xcd_tile((int)blockIdx.x, ntiles);
   const int bx = L % gx, t = L / gx, by = t % gy, bz = t / gy;
   const int ii = -2 + bx * 64 + (int)threadIdx.x;
   const int jj = -2 + by * 4 + (int)threadIdx.y;
   if (ii > d.ni + 3 || jj > d.nj + 3) return;
   const int n3 = d.n3, Z = d.sx * d.sy;
-  const int k0 = -2 + bz * kRnChunk, k1 = min(d.nk + 3, k0 + kRnChunk - 1);
+  const int k0 = -2 + bz * kc, k1 = min(d.nk + 3, k0 + kc - 1);
   // tangent mode: gradients below 1e-10 |dxinv| count as flat (no interface)
   const double flat2 = (val(verysmall) * 1.0e20) * (val(verysmall) * 1.0e20);
   const bool col_ok = ii >= -2 + ip && jj >= -2 + jp;
@@ -115,10 +115,11 @@ __global__ void __launch_bounds__(256) calrn_kernel(Dims d, T verysmall, int ip,
 template <class T>
 void calrn(const Dims d, double verysmall, int ip, int jp, int kp, const T* px, const T* py,
            const T* pz, T* rn) {
-  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4, gz = (d.sz + kRnChunk - 1) / kRnChunk;
+  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4;
+  const int kc = march_planes(gx * gy, d.sz, kRnChunk), gz = (d.sz + kc - 1) / kc;
   const int n = gx * gy * gz;
   calrn_kernel<T><<<dim3(n), dim3(64, 4, 1), 0, stream()>>>(d, T(verysmall), ip, jp, kp, px, py, pz,
-                                                            rn, gx, gy, xcd_arg(2, n));
+                                                            rn, gx, gy, xcd_arg(2, n), kc);
   FEL_CHECK(hipGetLastError());
 }
 
@@ -136,14 +137,14 @@ __global__ void __launch_bounds__(256) calrn4_kernel(Dims d, T verysmall, const 
                                                      const T* __restrict__ py,
                                                      const T* __restrict__ pz, T* __restrict__ r0,
                                                      T* __restrict__ r1, T* __restrict__ r2,
-                                                     T* __restrict__ r3, int gx, int gy) {
+                                                     T* __restrict__ r3, int gx, int gy, int kc) {
   const int L = (int)blockIdx.x;
   const int bx = L % gx, t = L / gx, by = t % gy, bz = t / gy;
   const int ii = -2 + bx * 64 + (int)threadIdx.x;
   const int jj = -2 + by * 4 + (int)threadIdx.y;
   if (ii > d.ni + 3 || jj > d.nj + 3) return;
   const int n3 = d.n3, X = 1, Y = d.sx;
-  const int k0 = -2 + bz * kRnChunk, k1 = min(d.nk + 3, k0 + kRnChunk - 1);
+  const int k0 = -2 + bz * kc, k1 = min(d.nk + 3, k0 + kc - 1);
   // tangent mode: gradients below 1e-10 |dxinv| count as flat (no interface)
   const double flat2 = (val(verysmall) * 1.0e20) * (val(verysmall) * 1.0e20);
   const bool xm = ii >= -1, ym = jj >= -1;  // the i-1 / j-1 neighbours exist
@@ -203,9 +204,10 @@ __global__ void __launch_bounds__(256) calrn4_kernel(Dims d, T verysmall, const 
 
 template <class T>
 void calrn4(const Dims d, double verysmall, const T* px, const T* py, const T* pz, T* const* rn) {
-  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4, gz = (d.sz + kRnChunk - 1) / kRnChunk;
+  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4;
+  const int kc = march_planes(gx * gy, d.sz, kRnChunk), gz = (d.sz + kc - 1) / kc;
   calrn4_kernel<T><<<dim3(gx * gy * gz), dim3(64, 4, 1), 0, stream()>>>(
-      d, T(verysmall), px, py, pz, rn[0], rn[1], rn[2], rn[3], gx, gy);
+      d, T(verysmall), px, py, pz, rn[0], rn[1], rn[2], rn[3], gx, gy, kc);
   FEL_CHECK(hipGetLastError());
 }
 
@@ -224,7 +226,7 @@ template <class T>
 __global__ void __launch_bounds__(512) calrn4_kap_kernel(
     Dims d, T verysmall, T dxinv, T dyinv, T dzinv, const T* __restrict__ px,
     const T* __restrict__ py, const T* __restrict__ pz, T* __restrict__ r0, T* __restrict__ r1,
-    T* __restrict__ r2, T* __restrict__ r3, T* __restrict__ rk, int gx, int gy) {
+    T* __restrict__ r2, T* __restrict__ r3, T* __restrict__ rk, int gx, int gy, int kc) {
   // [plane parity][rpp x, r12 x, r13 x, rpp y, r12 y, r23 y][row][lane]
   __shared__ T xs[2][6][kKapTy + 2][64];
   const int L = (int)blockIdx.x;
@@ -236,7 +238,7 @@ __global__ void __launch_bounds__(512) calrn4_kap_kernel(
   const bool vt = ii >= -2 && ii <= ni + 3 && jj >= -2 && jj <= nj + 3;
   const bool own = vt && tx >= 1 && tx <= kKapTx && ty >= 1 && ty <= kKapTy;
   const int n3 = d.n3, X = 1, Y = d.sx;
-  const int k0 = -2 + bz * kRnChunk, k1 = min(nk + 3, k0 + kRnChunk - 1);
+  const int k0 = -2 + bz * kc, k1 = min(nk + 3, k0 + kc - 1);
   const double flat2 = (val(verysmall) * 1.0e20) * (val(verysmall) * 1.0e20);
   const bool xm = ii >= -1, ym = jj >= -1;
   T* out[4] = {r0, r1, r2, r3};
@@ -345,10 +347,10 @@ template <class T>
 void calrn4_kap(const Dims d, double verysmall, double dxinv, double dyinv, double dzinv,
                 const T* px, const T* py, const T* pz, T* const* rn, T* rk) {
   const int gx = (d.sx + kKapTx - 1) / kKapTx, gy = (d.sy + kKapTy - 1) / kKapTy;
-  const int gz = (d.sz + kRnChunk - 1) / kRnChunk;
+  const int kc = march_planes(gx * gy, d.sz, kRnChunk, 2), gz = (d.sz + kc - 1) / kc;
   calrn4_kap_kernel<T><<<dim3(gx * gy * gz), dim3(64, kKapTy + 2, 1), 0, stream()>>>(
       d, T(verysmall), T(dxinv), T(dyinv), T(dzinv), px, py, pz, rn[0], rn[1], rn[2], rn[3], rk,
-      gx, gy);
+      gx, gy, kc);
   FEL_CHECK(hipGetLastError());
 }
 

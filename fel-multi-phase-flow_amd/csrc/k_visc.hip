@@ -109,13 +109,14 @@ template <class T>
 __global__ void __launch_bounds__(256) div_tensor_kernel(Dims d, T dxinv, T dyinv, T dzinv,
                                                          const T* __restrict__ tau,
                                                          T* __restrict__ vu, T* __restrict__ vv,
-                                                         T* __restrict__ vw, int gx, int gy) {
+                                                         T* __restrict__ vw, int gx, int gy,
+                                                         int kc) {
   const int L = (int)blockIdx.x;
   const int bx = L % gx, tt = L / gx, by = tt % gy, bz = tt / gy;
   const int ni = d.ni, nj = d.nj, nk = d.nk, n3 = d.n3;
   const int i = -2 + bx * 64 + (int)threadIdx.x, j = -2 + by * 4 + (int)threadIdx.y;
   if (i > ni + 3 || j > nj + 3) return;
-  const int k0 = -2 + bz * kDivChunk, k1 = min(nk + 3, k0 + kDivChunk - 1);
+  const int k0 = -2 + bz * kc, k1 = min(nk + 3, k0 + kc - 1);
   const T *t1 = tau, *t2 = tau + n3, *t3 = tau + 2 * n3, *t4 = tau + 3 * n3, *t5 = tau + 4 * n3,
           *t6 = tau + 5 * n3;
   const int X = 1, Y = d.sx, Z = d.sx * d.sy;
@@ -147,9 +148,10 @@ __global__ void __launch_bounds__(256) div_tensor_kernel(Dims d, T dxinv, T dyin
 template <class T>
 void div_tensor(const Dims d, double dxinv, double dyinv, double dzinv, const T* tau, T* vu,
                 T* vv, T* vw) {
-  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4, gz = (d.sz + kDivChunk - 1) / kDivChunk;
+  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4;
+  const int kc = march_planes(gx * gy, d.sz, kDivChunk), gz = (d.sz + kc - 1) / kc;
   div_tensor_kernel<T><<<dim3(gx * gy * gz), dim3(64, 4, 1), 0, stream()>>>(
-      d, T(dxinv), T(dyinv), T(dzinv), tau, vu, vv, vw, gx, gy);
+      d, T(dxinv), T(dyinv), T(dzinv), tau, vu, vv, vw, gx, gy, kc);
   FEL_CHECK(hipGetLastError());
 }
 
@@ -180,7 +182,8 @@ struct SijTau {
 constexpr int kSijChunk = 2;
 
 template <class T>
-__global__ void __launch_bounds__(256) sij_tau_kernel(Dims d, SijTau<T> a, int gx, int gy) {
+__global__ void __launch_bounds__(256) sij_tau_kernel(Dims d, SijTau<T> a, int gx, int gy,
+                                                      int kc) {
   const int L = (int)blockIdx.x;
   const int bx = L % gx, t = L / gx, by = t % gy, bz = t / gy;
   const int ni = d.ni, nj = d.nj, nk = d.nk;
@@ -188,7 +191,7 @@ __global__ void __launch_bounds__(256) sij_tau_kernel(Dims d, SijTau<T> a, int g
   const int j = -2 + by * 4 + (int)threadIdx.y;
   if (i > ni + 3 || j > nj + 3) return;
   const int n3 = d.n3, X = 1, Y = d.sx, Z = d.sx * d.sy;
-  const int k0 = -2 + bz * kSijChunk, k1 = min(nk + 3, k0 + kSijChunk - 1);
+  const int k0 = -2 + bz * kc, k1 = min(nk + 3, k0 + kc - 1);
   const T *u = a.u, *v = a.v, *w = a.w, *rmu = a.rmu;
   const bool xl = i >= -1, xr = i <= ni + 2, yl = j >= -1, yr = j <= nj + 2;
   const T q = T(0.25), h = T(0.5), two = T(2.0);
@@ -240,8 +243,9 @@ __global__ void __launch_bounds__(256) sij_tau_kernel(Dims d, SijTau<T> a, int g
 
 template <class T>
 void sij_tau(const Dims d, SijTau<T> a) {
-  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4, gz = (d.sz + kSijChunk - 1) / kSijChunk;
-  sij_tau_kernel<T><<<dim3(gx * gy * gz), dim3(64, 4, 1), 0, stream()>>>(d, a, gx, gy);
+  const int gx = (d.sx + 63) / 64, gy = (d.sy + 3) / 4;
+  const int kc = march_planes(gx * gy, d.sz, kSijChunk), gz = (d.sz + kc - 1) / kc;
+  sij_tau_kernel<T><<<dim3(gx * gy * gz), dim3(64, 4, 1), 0, stream()>>>(d, a, gx, gy, kc);
   FEL_CHECK(hipGetLastError());
 }
 

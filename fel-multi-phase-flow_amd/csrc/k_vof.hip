@@ -274,15 +274,6 @@ __global__ void __launch_bounds__(256) flux_interface_kernel(Dims d, FluxArgs<T>
   }
 }
 
-// Planes per thread of a marching launch of gxy blocks per plane over nz
-// planes: `most` where that leaves the chip full (2 blocks of 256 threads per
-// CU), fewer on smaller grids, whose time is one thread's serial march.
-inline int march_planes(int gxy, int nz, int most) {
-  int kc = most;
-  while (kc > 1 && gxy * ((nz + kc - 1) / kc) < 512) kc /= 2;
-  return kc;
-}
-
 template <class T, class P = PT<T>>
 void mthinc_flux(const Dims d, double dxinv, double dyinv, double dzinv, double dt,
                  MthincConst mc64, const P* phi, const T* phix, const T* phiy, const T* phiz,

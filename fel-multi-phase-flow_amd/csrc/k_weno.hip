@@ -113,7 +113,7 @@ __device__ __forceinline__ T weno_q(const T* q, T vel00) {
                -q[5] + q[6], vel00);
 }
 
-// Interior cells, k-marching: one thread per (i,j) column over kWenoK planes.
+// Interior cells, k-marching: one thread per (i,j) column over up to kWenoK planes.
 // The own column's u, v, w at k-3..k+3 live in register queues, so the
 // z-direction stencils load one new plane per step instead of seven; the
 // in-plane (x, y) stencils and the neighbour-column transport velocities are
@@ -130,12 +130,13 @@ __global__ void __launch_bounds__(256) weno_march_kernel(Dims d, T dxinv, T dyin
                                                          const T* __restrict__ v,
                                                          const T* __restrict__ w,
                                                          T* __restrict__ au, T* __restrict__ av,
-                                                         T* __restrict__ aw, int gx, int gy) {
+                                                         T* __restrict__ aw, int gx, int gy,
+                                                         int kc) {
   const int L = (int)blockIdx.x;
   const int bx = L % gx, t = L / gx, by = t % gy, bz = t / gy;
   const int i = 1 + bx * 64 + (int)threadIdx.x, j = 1 + by * 4 + (int)threadIdx.y;
   if (i > d.ni || j > d.nj) return;
-  const int k0 = 1 + bz * kWenoK, k1 = min(d.nk, k0 + kWenoK - 1);
+  const int k0 = 1 + bz * kc, k1 = min(d.nk, k0 + kc - 1);
   const int X = 1, Y = d.sx, Z = d.sx * d.sy;
   int c = d.ix(i, j, k0);
   T qu[7], qv[7], qw[7];
@@ -197,9 +198,10 @@ template <class T>
 void advect_weno5(const Dims d, double dxinv, double dyinv, double dzinv, const T* __restrict__ u,
                   const T* __restrict__ v, const T* __restrict__ w, T* __restrict__ au,
                   T* __restrict__ av, T* __restrict__ aw) {
-  const int gx = (d.ni + 63) / 64, gy = (d.nj + 3) / 4, gz = (d.nk + kWenoK - 1) / kWenoK;
+  const int gx = (d.ni + 63) / 64, gy = (d.nj + 3) / 4;
+  const int kc = march_planes(gx * gy, d.nk, kWenoK), gz = (d.nk + kc - 1) / kc;
   weno_march_kernel<T><<<dim3(gx * gy * gz), dim3(64, 4, 1), 0, stream()>>>(
-      d, T(dxinv), T(dyinv), T(dzinv), u, v, w, au, av, aw, gx, gy);
+      d, T(dxinv), T(dyinv), T(dzinv), u, v, w, au, av, aw, gx, gy, kc);
   FEL_CHECK(hipGetLastError());
   launch_shell(d, [=] __device__(int i, int j, int k) {
     const int c = d.ix(i, j, k);

@@ -44,3 +44,63 @@ def test_mthinc_flux_and_truncation_shapes(ni, nj, nk, flat):
     p = np.clip(g.interior(phin), 0.0, 1.0)
     bar = 4 / 27 * 2 * p.size * 1.2e-16 * p.sum() / (p * p * (1 - p)).sum() + 1e-15
     assert np.max(np.abs(a[-1] - b[-1])) <= bar
+
+
+class Resident:
+    """Arrays registered with the library for one test."""
+
+    def __init__(self, *arrays):
+        self.lib, self.arrays = H.gpu(), arrays
+
+    def __enter__(self):
+        for a in self.arrays:
+            self.lib.felgpu_register_(H.ctypes.c_void_p(a.ctypes.data),
+                                      H.ctypes.byref(H.ctypes.c_int64(a.nbytes)),
+                                      H.ctypes.byref(H.ctypes.c_int(1)))
+        return self
+
+    def fetch(self):
+        for a in self.arrays:
+            self.lib.felgpu_download_(H.ctypes.c_void_p(a.ctypes.data))
+
+    def __exit__(self, *exc):
+        for a in self.arrays:
+            self.lib.felgpu_unregister_(H.ctypes.c_void_p(a.ctypes.data))
+
+
+# sizes at which the marching kernels take 1, 2, 4 and (the normals) 16 planes
+MARCH = [(4, 4, 4), (61, 7, 13), (130, 40, 40), (70, 50, 160), (260, 124, 130)]
+
+
+@pytest.mark.parametrize("ni,nj,nk", MARCH)
+def test_marching_stencils_shapes(ni, nj, nk):
+    """Normals on four staggerings with their curvature, WENO5, and stress with
+    its divergence on resident arrays: bit for bit the oracle's."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    r = np.random.default_rng(ni * nj + nk)
+    head = [I(ni), I(nj), I(nk), D(1 / g.dx), D(1 / g.dy), D(1 / g.dz)]
+    grads = [r.standard_normal(g.shape) for _ in range(3)]
+    rn, kap = [g.zeros(3) for _ in range(4)], g.zeros(3)
+    vel, mu = [r.standard_normal(g.shape) for _ in range(3)], r.uniform(0.1, 1.0, g.shape)
+    adv, vis = [g.zeros() for _ in range(3)], [g.zeros() for _ in range(3)]
+    s, tau = g.zeros(6), g.zeros(6)
+    outs = rn + [kap] + adv + [s, tau] + vis
+
+    def calls(call):
+        for st, o in zip(((1, 1, 1), (0, 0, 1), (0, 1, 0), (1, 0, 0)), rn):
+            call("calrn", *head, *[I(v) for v in st], *grads, o)
+        call("calrkap", *head, *rn, kap)
+        call("cal_advu_weno5", *head, *vel, *adv)
+        call("calsij", *head, *vel, s)
+        call("cal_arith_tau", *head[:3], s, mu, tau)
+        call("cal_div_tensor", *head, tau, *vis)
+
+    calls(H.call_oracle)
+    want = [o.copy() for o in outs]
+    for o in outs:
+        o[...] = 0.0
+    with Resident(*grads, *vel, mu, *outs) as res:
+        calls(H.call_gpu)
+        res.fetch()
+    for a, b in zip(want, outs):
+        assert np.array_equal(a, b)
