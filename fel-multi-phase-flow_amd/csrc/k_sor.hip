@@ -140,13 +140,38 @@ constexpr int kKB = 1;
 // R00I: the face density of each update is formed in the launch from rho and
 // rhon with the expression of the per-solve table (the same bits), for the
 // allocation-free entry point, which keeps no table.
-// One cell's update of component COMP (srcs/solu_sor4.f:131-175) at c, with
-// the swept component's x neighbours xm = F[c-X], xp = F[c+X] supplied by
+// FORM: how the ghosts are to be read.  kStored: as they are (a refresh launch
+// ran before this pair, or the caller's ghosts).  Otherwise the stored ghosts
+// are the periodic images of every component (and the wall rows), kept by the
+// in-launch images, and what the refresh of the swept component leaves
+// different -- bndu's shifted sources, which set u's ghost column 0 to u(ni+1)
+// and w's ghost plane 0 to w(nk+1) (srcs/bndu.f:107-109,144-146), undone by
+// bnd_periodic for the swept component only -- is read from there: kFirst,
+// the first pair of a component's sweep, which sees the ghosts the previous
+// component's refresh left; kLater, the other pairs.
+enum SorForm { kStored, kFirst, kLater };
+
+// Reads u(c-X) (and rows or planes beside it) in the v and w equations.
+template <int COMP, int FORM>
+__device__ __forceinline__ constexpr bool shifted_u() {
+  return (COMP == 1 && FORM == kLater) || (COMP == 2 && FORM != kStored);
+}
+// Reads w(c-Z) in the u and v equations.
+template <int COMP, int FORM>
+__device__ __forceinline__ constexpr bool shifted_w() {
+  return (COMP == 0 && FORM == kLater) || (COMP == 1 && FORM != kStored);
+}
+
+// One cell's update of component COMP (srcs/solu_sor4.f:131-175) at c = (i,j,k),
+// with the swept component's x neighbours xm = F[c-X], xp = F[c+X] supplied by
 // the caller; returns the new value (not stored) and adds du^2 to e.
-template <int COMP, bool ONFLY, class T, bool R00I>
-__device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c, int ridx, T xm,
-                                      T xp, double& e) {
+template <int COMP, bool ONFLY, int FORM, class T, bool R00I>
+__device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c, int i, int k,
+                                      int ridx, T xm, T xp, double& e) {
   const int X = 1, Y = d.sx, Z = d.sx * d.sy;
+  const int UX = shifted_u<COMP, FORM>() && i == 1 ? d.ni : -X;        // u(c-X)
+  const int WZ = shifted_w<COMP, FORM>() && k == 1 ? d.nk * Z : -Z;    // w(c-Z)
+  const int FZ = COMP == 2 && FORM == kFirst && k == 1 ? d.nk * Z : -Z;  // own (c-Z)
   T cf[15];
   if (ONFLY) {
     if (COMP == 0) coef_u(d, a.sc, a.rmu, c, cf);
@@ -174,20 +199,20 @@ __device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c,
     visn = (+A(cf[4]) * A(un[c - Z]) + A(cf[2]) * A(un[c - Y]) + A(cf[0]) * A(xm) +
                  A(cf[1]) * A(xp) + A(cf[3]) * A(un[c + Y]) + A(cf[5]) * A(un[c + Z]) +
                  A(cf[7]) * A(vn[c - Y]) + A(cf[8]) * A(vn[c + X - Y]) + A(cf[9]) * A(vn[c]) +
-                 A(cf[10]) * A(vn[c + X]) + A(cf[11]) * A(wn[c - Z]) + A(cf[12]) * A(wn[c + X - Z]) +
+                 A(cf[10]) * A(vn[c + X]) + A(cf[11]) * A(wn[c + WZ]) + A(cf[12]) * A(wn[c + X + WZ]) +
                  A(cf[13]) * A(wn[c]) + A(cf[14]) * A(wn[c + X])) /
                 A(r00);
   } else if (COMP == 1) {
     visn = (+A(cf[4]) * A(vn[c - Z]) + A(cf[2]) * A(vn[c - Y]) + A(cf[0]) * A(xm) +
                  A(cf[1]) * A(xp) + A(cf[3]) * A(vn[c + Y]) + A(cf[5]) * A(vn[c + Z]) +
-                 A(cf[7]) * A(un[c - X]) + A(cf[9]) * A(un[c]) + A(cf[8]) * A(un[c - X + Y]) +
-                 A(cf[10]) * A(un[c + Y]) + A(cf[11]) * A(wn[c - Z]) + A(cf[12]) * A(wn[c + Y - Z]) +
+                 A(cf[7]) * A(un[c + UX]) + A(cf[9]) * A(un[c]) + A(cf[8]) * A(un[c + UX + Y]) +
+                 A(cf[10]) * A(un[c + Y]) + A(cf[11]) * A(wn[c + WZ]) + A(cf[12]) * A(wn[c + Y + WZ]) +
                  A(cf[13]) * A(wn[c]) + A(cf[14]) * A(wn[c + Y])) /
                 A(r00);
   } else {
-    visn = (+A(cf[4]) * A(wn[c - Z]) + A(cf[2]) * A(wn[c - Y]) + A(cf[0]) * A(xm) +
+    visn = (+A(cf[4]) * A(wn[c + FZ]) + A(cf[2]) * A(wn[c - Y]) + A(cf[0]) * A(xm) +
                  A(cf[1]) * A(xp) + A(cf[3]) * A(wn[c + Y]) + A(cf[5]) * A(wn[c + Z]) +
-                 A(cf[7]) * A(un[c - X]) + A(cf[9]) * A(un[c]) + A(cf[8]) * A(un[c - X + Z]) +
+                 A(cf[7]) * A(un[c + UX]) + A(cf[9]) * A(un[c]) + A(cf[8]) * A(un[c + UX + Z]) +
                  A(cf[10]) * A(un[c + Z]) + A(cf[11]) * A(vn[c - Y]) + A(cf[13]) * A(vn[c]) +
                  A(cf[12]) * A(vn[c - Y + Z]) + A(cf[14]) * A(vn[c + Z])) /
                 A(r00);
@@ -205,23 +230,11 @@ __device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c,
   return nv;
 }
 
-template <int COMP, bool ONFLY, bool FUSE, class T, bool R00I = false>
-__device__ __forceinline__ void sor_pair_body(const Dims& d, const SorArgs<T>& a, int is, int js,
-                                              int ks, int jend, int gx, int gy, int ntiles,
-                                              double* part);
-
-
-template <int COMP, bool ONFLY, bool FUSE, class T, bool R00I = false>
-__global__ void __launch_bounds__(512) sor_pair_kernel(Dims d, SorArgs<T> a, int is, int js, int ks,
+// FORM != kStored: the pair's ghost images are written by the launch.
+template <int COMP, bool ONFLY, int FORM, class T, bool R00I = false>
+__global__ void __launch_bounds__(512, ONFLY && sizeof(T) == 8 ? 8 : 1) sor_pair_kernel(Dims d, SorArgs<T> a, int is, int js, int ks,
                                                        int jend, int gx, int gy, int ntiles,
                                                        double* part) {
-  sor_pair_body<COMP, ONFLY, FUSE, T, R00I>(d, a, is, js, ks, jend, gx, gy, ntiles, part);
-}
-
-template <int COMP, bool ONFLY, bool FUSE, class T, bool R00I>
-__device__ __forceinline__ void sor_pair_body(const Dims& d, const SorArgs<T>& a, int is, int js,
-                                              int ks, int jend, int gx, int gy, int ntiles,
-                                              double* part) {
   const int L = xcd_tile((int)blockIdx.x, ntiles);
   const int bx = L % gx, tt = L / gx, by = tt % gy, bz = tt / gy;
   double e = 0.0;
@@ -237,9 +250,11 @@ __device__ __forceinline__ void sor_pair_body(const Dims& d, const SorArgs<T>& a
     const int c = d.ix(i, j, k);
     const int ridx = r00_index(d, ii, by * (int)blockDim.y + (int)threadIdx.y, k);
     T* F = COMP == 0 ? a.un : (COMP == 1 ? a.vn : a.wn);
-    const T nv = sor_cell<COMP, ONFLY, T, R00I>(d, a, c, ridx, F[c - X], F[c + X], e);
+    // u's own ghost column 0 before its first pair: u(ni+1)
+    const T xm = F[COMP == 0 && FORM == kFirst && i == 1 ? c + d.ni : c - X];
+    const T nv = sor_cell<COMP, ONFLY, FORM, T, R00I>(d, a, c, i, k, ridx, xm, F[c + X], e);
     put_update(F, c, nv);
-    if (FUSE) write_images<COMP>(d, a, F, i, j, k, nv);
+    if (FORM != kStored) write_images<COMP>(d, a, F, i, j, k, nv);
   }
   }
   // block sum of du^2 in a fixed order
@@ -301,7 +316,7 @@ __global__ void __launch_bounds__(512) sor_pair12_kernel(Dims d, SorArgs<T> a1, 
   T nv1 = T(0.0);
   if (row) {
     const int c = d.ix(i1, j, k);
-    nv1 = sor_cell<COMP, ONFLY, T, false>(d, a1, c, ridx, F[c - X], F[c + X], e1);
+    nv1 = sor_cell<COMP, ONFLY, kLater, T, false>(d, a1, c, i1, k, ridx, F[c - X], F[c + X], e1);
     put_update(F, c, nv1);
     write_images<COMP>(d, a1, F, i1, j, k, nv1);
   }
@@ -317,7 +332,7 @@ __global__ void __launch_bounds__(512) sor_pair12_kernel(Dims d, SorArgs<T> a1, 
       xm = s1[t > 0 ? t - 1 : hx - 1];
       xp = s1[t];
     }
-    const T nv2 = sor_cell<COMP, ONFLY, T, false>(d, a2, c, ridx, xm, xp, e2);
+    const T nv2 = sor_cell<COMP, ONFLY, kLater, T, false>(d, a2, c, i2, k, ridx, xm, xp, e2);
     put_update(F, c, nv2);
     write_images<COMP>(d, a2, F, i2, j, k, nv2);
   }
@@ -383,7 +398,7 @@ struct SorResult {
 };
 
 template <int COMP, class T>
-void launch_pair(bool onfly, bool fuse, dim3 grid, dim3 block, const Dims& d, const SorArgs<T>& a,
+void launch_pair(bool onfly, int form, dim3 grid, dim3 block, const Dims& d, const SorArgs<T>& a,
                  int p, int jend, int gx, int gy, int nt, double* pp, hipEvent_t e0,
                  hipEvent_t e1) {
   hipStream_t s = stream();
@@ -396,18 +411,19 @@ void launch_pair(bool onfly, bool fuse, dim3 grid, dim3 block, const Dims& d, co
     hipExtLaunchKernelGGL(kernel, grid, block, 0, s, e0, e1, 0, d, ap, kIs[p], kJs[p], kKs[p],
                           jend, gx, gy, nt, pp);
   };
+  auto by_form = [&](auto onfly_c, auto r00i_c) {
+    constexpr bool of = decltype(onfly_c)::value, ri = decltype(r00i_c)::value;
+    if (form == kStored) go(sor_pair_kernel<COMP, of, kStored, T, ri>);
+    else if (form == kFirst) go(sor_pair_kernel<COMP, of, kFirst, T, ri>);
+    else go(sor_pair_kernel<COMP, of, kLater, T, ri>);
+  };
   if (r00i) {
     // the allocation-free form: coefficients from the viscosity, FP64 only
-    if constexpr (std::is_same_v<T, double>) {
-      if (fuse) go(sor_pair_kernel<COMP, true, true, T, true>);
-      else go(sor_pair_kernel<COMP, true, false, T, true>);
-    }
+    if constexpr (std::is_same_v<T, double>) by_form(std::true_type{}, std::true_type{});
     return;
   }
-  if (onfly && fuse) go(sor_pair_kernel<COMP, true, true, T>);
-  else if (onfly) go(sor_pair_kernel<COMP, true, false, T>);
-  else if (fuse) go(sor_pair_kernel<COMP, false, true, T>);
-  else go(sor_pair_kernel<COMP, false, false, T>);
+  if (onfly) by_form(std::true_type{}, std::false_type{});
+  else by_form(std::false_type{}, std::false_type{});
 }
 
 // Whether pairs 1 and 2 run as one launch (sor_pair12_kernel): even ni and
@@ -576,10 +592,16 @@ SorResult sor4(const Dims d, SorArgs<T> a, bool onfly, bool lo, bool hi, double 
           FEL_CHECK(hipGetLastError());
           continue;
         }
-        // Pairs after the first write the swept component's ghost images
-        // themselves (write_images); the refresh after the first pair also
-        // rewrites the other components' ghosts, so it stays a launch.
-        const bool fuse = fuse_ok && p > 0;
+        // Pairs write the swept component's ghost images themselves
+        // (write_images) and read the other components' ghosts by SorForm.
+        // The first pair of the solve sees the ghosts as the caller left
+        // them; the refresh launch after it makes them the images the rest
+        // of the solve keeps, up to w's, which stay w(nk+1) in plane 0 until
+        // the refresh after w's first pair (two such launches per solve
+        // instead of one per component and sweep: 21 us each at
+        // 512x256x128, a launch gap on small grids).
+        const int form = !fuse_ok || (p == 0 && comp == 0 && lp == 0) ? kStored
+                         : (p == 0 ? kFirst : kLater);
         const int nt = xcd_arg(1, nb);
         // The colour-pair timer: with pairs 1 and 2 joined, pair 3 (pair 0
         // is followed by a refresh launch and not timed); with fused images
@@ -594,18 +616,18 @@ SorResult sor4(const Dims d, SorArgs<T> a, bool onfly, bool lo, bool hi, double 
         } else {
           prof_launch_events(3, true, true, 1, &e0, &e1);
         }
-        if (comp == 0) launch_pair<0, T>(onfly, fuse, grid, block, d, a, p, jend, gx, gy, nt, pp, e0, e1);
-        if (comp == 1) launch_pair<1, T>(onfly, fuse, grid, block, d, a, p, jend, gx, gy, nt, pp, e0, e1);
-        if (comp == 2) launch_pair<2, T>(onfly, fuse, grid, block, d, a, p, jend, gx, gy, nt, pp, e0, e1);
+        if (comp == 0) launch_pair<0, T>(onfly, form, grid, block, d, a, p, jend, gx, gy, nt, pp, e0, e1);
+        if (comp == 1) launch_pair<1, T>(onfly, form, grid, block, d, a, p, jend, gx, gy, nt, pp, e0, e1);
+        if (comp == 2) launch_pair<2, T>(onfly, form, grid, block, d, a, p, jend, gx, gy, nt, pp, e0, e1);
         FEL_CHECK(hipGetLastError());
-        if (!fuse) {
+        if (form == kStored || (fuse_ok && lp == 0 && comp == 2 && p == 0)) {
           // After the first pair of a component's sweep only that component
           // changes, and bndu's ghosts of the other two are functions of their
           // unchanged interiors: rewriting them would store the same values.
           // With fused images the deep wall rows, read by no stencil of the
           // solve, are left to the refreshes after the last sweep.
           bc_fused<T, P>(d, a.un, a.vn, a.wn, uwall, dy, l1, l2, phi, lo, hi, comp,
-                         p == 0 ? 7 : (1 << comp), fuse_ok);
+                         p == 0 && form == kStored ? 7 : (1 << comp), fuse_ok);
         }
       }
     }

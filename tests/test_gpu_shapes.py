@@ -104,3 +104,39 @@ def test_marching_stencils_shapes(ni, nj, nk):
         res.fetch()
     for a, b in zip(want, outs):
         assert np.array_equal(a, b)
+
+
+# even x and z (ghost images in the launches: the smallest grid, one and several
+# blocks a row) and an odd size of each (refresh launches)
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (66, 7, 18), (130, 9, 6), (33, 8, 10), (8, 5, 9)])
+@pytest.mark.parametrize("resident", [False, True], ids=["coefficients", "viscosity"])
+def test_viscous_solve_with_any_ghosts(ni, nj, nk, resident):
+    """solu_sor4 from ghosts that are no periodic images: the values that its
+    pairs read through bndu's shifted sources are the ones the refreshes of the
+    oracle leave, bit for bit, whether the coefficients are arrays or formed
+    from the viscosity."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    r = np.random.default_rng(ni * nj + nk)
+    head = [I(ni), I(nj), I(nk)]
+    rmu, rho, rhon, phi, l1, l2 = (r.uniform(0.05, 1.0, g.shape) for _ in range(6))
+    src = [r.standard_normal(g.shape) for _ in range(3)]
+    start = [r.standard_normal(g.shape) for _ in range(3)]
+
+    def solve(call, coef, uvw):
+        call("cal_arith_coef_vis", *head, D(1 / g.dx), D(1 / g.dy), D(1 / g.dz), rmu, *coef)
+        call("solu_sor4", I(0), I(0), np.full(6, -1, np.int32), I(1), *head,
+             np.zeros(8, np.int32), np.zeros(8), np.zeros(8), I(1), I(0), D(0.01), rho, rhon,
+             *coef, *src, *uvw, D(0.25), D(g.dy), l1, l2, phi)
+
+    want, got = [x.copy() for x in start], [x.copy() for x in start]
+    solve(H.call_oracle, [g.zeros() for _ in range(45)], want)
+    coef = [g.zeros() for _ in range(45)]
+    if resident:
+        with Resident(rmu, rho, rhon, phi, l1, l2, *src, *coef, *got) as res:
+            solve(H.call_gpu, coef, got)
+            for a in got:
+                res.lib.felgpu_download_(H.ctypes.c_void_p(a.ctypes.data))
+    else:
+        solve(H.call_gpu, coef, got)
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
