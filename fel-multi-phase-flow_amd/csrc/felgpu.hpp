@@ -407,8 +407,7 @@ inline void launch_box(const Box& b, F f) {
 // Planes per thread of a kernel that marches in k, gxy blocks per layer of
 // threads over nz planes: `most` where that leaves the chip full (2 blocks per
 // CU), fewer (`least` at the lowest) on smaller grids, whose time is one
-// thread's serial march (32x8x32, FP64: WENO5 27 -> 13 us with 1 plane instead
-// of 4, the normals 47 -> 17 us with 2 instead of 16).
+// thread's serial march (a whole 32x8x32 step in FP64: 851 -> 822 us).
 inline int march_planes(int gxy, int nz, int most, int least = 1) {
   int kc = most;
   while (kc > least && gxy * ((nz + kc - 1) / kc) < 512) kc /= 2;

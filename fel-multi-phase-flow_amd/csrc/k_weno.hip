@@ -5,6 +5,7 @@
 // component; the ghost shell is zeroed (the reference's clearing pass,
 // cal_advu_weno5.f:44-52), so the outputs are written exactly once.
 #include <cstdlib>
+#include <type_traits>
 #include <vector>
 
 #include "felgpu.hpp"
@@ -25,10 +26,23 @@ namespace fel {
 // far below the FP32 mode's accuracy bar and which replaces a ten-instruction
 // division sequence in a compute-bound kernel.  The weight sums are floored
 // at 1e-30 and, after the scaling, lie far above the smallest normal float.
-template <class T>
-__device__ __forceinline__ T weight_rcp(T x) {
-  if constexpr (is_f32<T>) return __builtin_amdgcn_rcpf(x);
-  else return T(1.0) / x;
+// FAST (FP64): the quotient by Newton's iteration from the hardware reciprocal
+// with the final residual correction (Markstein), which is the correctly
+// rounded 1/x where no step leaves the normal range; the weight sums are at
+// least 1e-80, and one of 1e300 or more (or NaN) sets `odd`.
+template <bool FAST, class T>
+__device__ __forceinline__ T weight_rcp(T x, bool& odd) {
+  if constexpr (is_f32<T>) {
+    return __builtin_amdgcn_rcpf(x);
+  } else if constexpr (FAST) {
+    odd |= !(x < 1.0e300);
+    T r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(fma(-x, r, 1.0), r, r);
+  } else {
+    return T(1.0) / x;
+  }
 }
 
 // One upwind-biased side of srcs/weno5.h: w1*df1 + w2*df2 + w3*df3 of the
@@ -37,23 +51,30 @@ __device__ __forceinline__ T weight_rcp(T x) {
 // dfm3) -- with the candidate derivatives from those differences and the
 // smoothness indicators from their scaled copies (s5, s3, s1, t1, t3);
 // expressions in the reference's order.
+// p x + y with p a power of two, where the reference rounds p x and then the
+// sum: p x is exact, so one fused operation gives the same bits.
 template <class T>
+__device__ __forceinline__ T pow2_fma(double p, T x, T y) {
+  if constexpr (std::is_floating_point_v<T>) return fma(T(p), x, y);
+  else return x * T(p) + y;
+}
+
+template <bool FAST, class T>
 __device__ __forceinline__ T weno_side(T d5, T d3, T d1, T e1, T e3, T s5, T s3, T s1, T t1,
-                                       T t3) {
-  const T c2 = T(2.0), c3 = T(3.0), c4 = T(4.0), c5 = T(5.0), c7 = T(7.0), c11 = T(11.0),
-          c13 = T(13.0);
-  const T df_1 = d5 * c2 - d3 * c7 + d1 * c11;
-  const T df_2 = -d3 + d1 * c5 + e1 * c2;
-  const T df_3 = d1 * c2 + e1 * c5 - e3;
+                                       T t3, bool& odd) {
+  const T c3 = T(3.0), c5 = T(5.0), c7 = T(7.0), c11 = T(11.0), c13 = T(13.0);
+  const T df_1 = pow2_fma(2.0, d5, -(d3 * c7)) + d1 * c11;
+  const T df_2 = pow2_fma(2.0, e1, -d3 + d1 * c5);
+  const T df_3 = pow2_fma(2.0, d1, e1 * c5) - e3;
   T a, b;
-  a = s5 - s3 * c2 + s1;
-  b = s5 - s3 * c4 + s1 * c3;
+  a = pow2_fma(-2.0, s3, s5) + s1;
+  b = pow2_fma(-4.0, s3, s5) + s1 * c3;
   const T sm_1 = a * a * c13 + b * b * c3;
-  a = s3 - s1 * c2 + t1;
+  a = pow2_fma(-2.0, s1, s3) + t1;
   b = s3 - t1;
   const T sm_2 = a * a * c13 + b * b * c3;
-  a = s1 - t1 * c2 + t3;
-  b = s1 * c3 - t1 * c4 + t3;
+  a = pow2_fma(-2.0, t1, s1) + t3;
+  b = pow2_fma(-4.0, t1, s1 * c3) + t3;
   const T sm_3 = a * a * c13 + b * b * c3;
   T a_1 = sm_2 * sm_3, a_2 = sm_1 * sm_3, a_3 = sm_1 * sm_2;
   a_1 = a_1 * a_1;
@@ -61,68 +82,154 @@ __device__ __forceinline__ T weno_side(T d5, T d3, T d1, T e1, T e3, T s5, T s3,
   a_3 = a_3 * a_3;
   a_2 = a_2 * T(6.0);
   a_3 = a_3 * c3;
-  const T deninv = weight_rcp(a_1 + a_2 + a_3 + guard<T>(1.0e-80));
+  const T deninv = weight_rcp<FAST>(a_1 + a_2 + a_3 + guard<T>(1.0e-80), odd);
   const T w_1 = a_1 * deninv, w_3 = a_3 * deninv;
   const T w_2 = T(1.0) - w_1 - w_3;
   return w_1 * df_1 + w_2 * df_2 + w_3 * df_3;
 }
 
 // srcs/weno5.h:24-71: (velm1 * m side + velp1 * p side) / 12 with velm1 =
-// vel + |vel| and velp1 = vel - |vel|.  For vel != 0 one of the two factors
-// is an exact zero and its side is not evaluated: the sum is the other
-// term's value, the same bits (up to the sign of a zero result), and in the
-// tangent mode the zero factor's derivative is zero too.  vel = 0 (or NaN)
-// evaluates both sides as written.
-template <class T>
-__device__ __forceinline__ T weno5(T dfm5, T dfm3, T dfm1, T dfp1, T dfp3, T dfp5, T vel00) {
-  T m5 = dfm5, m3 = dfm3, m1 = dfm1, p1 = dfp1, p3 = dfp3, p5 = dfp5;
+// vel + |vel| and velp1 = vel - |vel|, vel = vel4 / 4, from the values
+// f(-3..3).  For vel != 0 one of the two factors is an exact zero and its side
+// is not evaluated: the sum is the other term's value, the same bits (up to
+// the sign of a zero result), and in the tangent mode the zero factor's
+// derivative is zero too.  vel = 0 (or NaN) evaluates both sides as written.
+//
+// The p side of f is minus the m side of its mirror image, sign for sign, and
+// both factors are 2 |vel| up to that sign.  So the upwind half of the values
+// is selected per lane and one polynomial is evaluated: a branch on the sign
+// runs both sides, one after the other, in every wavefront whose 64 cells hold
+// both signs.  The powers of two in 2 |vel| = |vel4| / 2 go into the constant.
+//
+// FAST: without branches; for vel = 0 the m side stands for both, which is the
+// same zero while both sides are finite.  `odd` is set where they may not be:
+// the m side sets it through its weights' sum, and of the values that only the
+// p side reads, or reads twice as often, f(2) and f(3) are looked at here.
+template <bool FAST, class T>
+__device__ __forceinline__ T weno_up(T fm3, T fm2, T fm1, T f0, T fp1, T fp2, bool& odd) {
+  const T d5 = fm2 - fm3, d3 = fm1 - fm2, d1 = f0 - fm1, e1 = fp1 - f0, e3 = fp2 - fp1;
   if constexpr (is_f32<T>) {
-    const T sc = fmax(fmax(fmax(fabs(m5), fabs(m3)), fmax(fabs(m1), fabs(p1))),
-                      fmax(fabs(p3), fabs(p5)));
+    const T mx = fmax(fmax(fmax(fabs(d5), fabs(d3)), fmax(fabs(d1), fabs(e1))), fabs(e3));
     // scale by the exact power of two that brings the largest difference to
-    // [1, 2): the weights are invariant to it, and unlike 1/sc (which
-    // overflows for sc below ~2.9e-39) it stays finite for subnormal sc
-    const int e = sc > T(0.0) ? ilogbf(sc) : 0;
-    m5 = ldexpf(m5, -e); m3 = ldexpf(m3, -e); m1 = ldexpf(m1, -e);
-    p1 = ldexpf(p1, -e); p3 = ldexpf(p3, -e); p5 = ldexpf(p5, -e);
+    // [1, 2): the weights are invariant to it, and unlike 1/mx (which
+    // overflows for mx below ~2.9e-39) it stays finite for subnormal mx
+    const int e = mx > T(0.0) ? -ilogbf(mx) : 0;
+    return weno_side<FAST>(d5, d3, d1, e1, e3, T(ldexpf(d5, e)), T(ldexpf(d3, e)),
+                           T(ldexpf(d1, e)), T(ldexpf(e1, e)), T(ldexpf(e3, e)), odd);
+  } else {
+    return weno_side<FAST>(d5, d3, d1, e1, e3, d5, d3, d1, e1, e3, odd);
   }
-  const T velab = fabs(vel00);
-  const T velm1 = vel00 + velab, velp1 = vel00 - velab;
-  const T r12 = T(1.0) / T(12.0);
-  if (vel00 > T(0.0))
-    return (velm1 * weno_side(dfm5, dfm3, dfm1, dfp1, dfp3, m5, m3, m1, p1, p3)) * r12;
-  if (vel00 < T(0.0))
-    return (velp1 * weno_side(dfp5, dfp3, dfp1, dfm1, dfm3, p5, p3, p1, m1, m3)) * r12;
-  return (velm1 * weno_side(dfm5, dfm3, dfm1, dfp1, dfp3, m5, m3, m1, p1, p3) +
-          velp1 * weno_side(dfp5, dfp3, dfp1, dfm1, dfm3, p5, p3, p1, m1, m3)) *
-         r12;
+}
+
+template <bool FAST, class T>
+__device__ __forceinline__ T weno5(T fm3, T fm2, T fm1, T f0, T fp1, T fp2, T fp3, T vel4,
+                                   bool& odd) {
+  const T r12 = T(1.0) / T(12.0), r24 = T(0.5) * r12;
+  const bool down = vel4 < T(0.0);
+  const T side = weno_up<FAST>(down ? fp3 : fm3, down ? fp2 : fm2, down ? fp1 : fm1, f0,
+                               down ? fm1 : fp1, down ? fm2 : fp2, odd);
+  if constexpr (FAST) {
+    odd |= !(fabs(vel4) > T(0.0)) && !(fabs(fp2) < T(1.0e30) && fabs(fp3) < T(1.0e30));
+    return (fabs(vel4) * side) * r24;
+  } else {
+    if (down || vel4 > T(0.0)) return (fabs(vel4) * side) * r24;
+    const T vel00 = vel4 * T(0.25), velab = fabs(vel00);
+    const T velm1 = vel00 + velab, velp1 = vel00 - velab;
+    return (velm1 * side - velp1 * weno_up<FAST>(fp3, fp2, fp1, f0, fm1, fm2, odd)) * r12;
+  }
+}
+
+// The value at a byte offset from a row's start.  The rows are the same for
+// all lanes of a wavefront (64 cells along x), so their addresses are scalar
+// and a load needs no vector address arithmetic.
+template <class T>
+__device__ __forceinline__ T at(const T* row, uint32_t off) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(row) + off);
 }
 
 template <class T>
-__device__ __forceinline__ T weno_dir(const T* __restrict__ f, int c, int st, T vel00) {
-  const T fm3 = f[c - 3 * st], fm2 = f[c - 2 * st], fm1 = f[c - st], f0 = f[c];
-  const T fp1 = f[c + st], fp2 = f[c + 2 * st], fp3 = f[c + 3 * st];
-  return weno5(-fm3 + fm2, -fm2 + fm1, -fm1 + f0, -f0 + fp1, -fp1 + fp2, -fp2 + fp3, vel00);
+__device__ __forceinline__ void put(T* row, uint32_t off, T x) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(row) + off) = x;
+}
+
+template <bool FAST, class T>
+__device__ __forceinline__ T weno_dir(const T* __restrict__ f, uint32_t off, ptrdiff_t st, T vel4,
+                                      bool& odd) {
+  return weno5<FAST>(at(f - 3 * st, off), at(f - 2 * st, off), at(f - st, off), at(f, off),
+                     at(f + st, off), at(f + 2 * st, off), at(f + 3 * st, off), vel4, odd);
 }
 
 // The WENO5 derivative from a register queue f(k-3..k+3) of the cell's own
-// column (the z direction), same differences as weno_dir.
-template <class T>
-__device__ __forceinline__ T weno_q(const T* q, T vel00) {
-  return weno5(-q[0] + q[1], -q[1] + q[2], -q[2] + q[3], -q[3] + q[4], -q[4] + q[5],
-               -q[5] + q[6], vel00);
+// column (the z direction).
+template <bool FAST, class T>
+__device__ __forceinline__ T weno_q(const T* q, T vel4, bool& odd) {
+  return weno5<FAST>(q[0], q[1], q[2], q[3], q[4], q[5], q[6], vel4, odd);
 }
 
-// Interior cells, k-marching: one thread per (i,j) column over up to kWenoK planes.
-// The own column's u, v, w at k-3..k+3 live in register queues, so the
-// z-direction stencils load one new plane per step instead of seven; the
-// in-plane (x, y) stencils and the neighbour-column transport velocities are
-// loaded from the same plane, which the block's other lanes share in cache.
-// Every value entering the arithmetic is the same double as in the
-// one-thread-per-cell form, so the results are identical.
-// Planes per thread (measured at 512x256x128: 745 us in FP64 and 407 us in
-// FP32 with 4, against 759 and 430 with 16; 2 and 8 within 3%).
-constexpr int kWenoK = 4;
+// Interior cells, k-marching: one thread per (i,j) column of one component
+// over up to kWenoK planes.  The own column's component at k-3..k+3 lives in a
+// register queue, so the z-direction stencil loads one new plane per step
+// instead of seven; the in-plane (x, y) stencils and the transport velocities
+// are loaded from the same plane, which the block's other lanes share in cache.
+//
+// Bound by the FP64 units: about 95 operations a derivative, issued in 75% of
+// the cycles.  Measured at 512x128x256 with velocities of both signs: 606 us
+// in FP64, 342 us in FP32 and 1.52 ms in the tangent mode; a branch per side and all components in one
+// thread took 810 us, 464 us and 2.10 ms, the one polynomial per lane alone
+// 657 us in FP64.  One
+// component per thread holds 93 registers instead of 124, which keeps 5
+// wavefronts on a SIMD instead of 4 and triples the threads of a small grid
+// (7.6 -> 4.6 us at 32x8x32); the three columns of one place run side by side
+// on one XCD, whose L2 they share.  Planes per thread: 633, 606 and 606 us
+// with 4, 8 and 16.
+constexpr int kWenoK = 8;
+
+template <int COMP, class T>
+__device__ __forceinline__ void weno_column(ptrdiff_t Y, ptrdiff_t Z, T dxinv, T dyinv, T dzinv,
+                                            const T* __restrict__ u, const T* __restrict__ v,
+                                            const T* __restrict__ w, T* __restrict__ out,
+                                            uint32_t off, int planes) {
+  const ptrdiff_t X = 1;
+  // towards the component's face
+  const ptrdiff_t S = COMP == 0 ? X : (COMP == 1 ? Y : Z);
+  const T* __restrict__ f = COMP == 0 ? u : (COMP == 1 ? v : w);
+  T q[7];
+#pragma unroll
+  for (int m = 0; m < 6; m++) q[m + 1] = at(f + (m - 3) * Z, off);
+  for (int n = 0; n < planes; n++, f += Z, u += Z, v += Z, w += Z, out += Z) {
+    // one address register: the lanes' offset is made opaque, or its widening
+    // to 64 bits leaves the loop and every load adds it to the row again
+    uint32_t o = off;
+    asm volatile("" : "+v"(o));
+#pragma unroll
+    for (int m = 0; m < 6; m++) q[m] = q[m + 1];
+    q[6] = at(f + 3 * Z, o);
+    // The transport velocity is the mean of two face means; its halvings are
+    // exact and left to weno5 (sums of two sums, four times the mean).
+    // (srcs/cal_advu_weno5.f:80-120, 147-187, 214-254)
+    auto cell = [&](auto fast, bool& odd) {
+      constexpr bool F = decltype(fast)::value;
+      const T vx = COMP == 0 ? (at(u - X, o) + q[3]) + (q[3] + at(u + X, o))
+                             : (at(u - X, o) + at(u - X + S, o)) + (at(u, o) + at(u + S, o));
+      const T vy = COMP == 1 ? (at(v - Y, o) + q[3]) + (q[3] + at(v + Y, o))
+                             : (at(v - Y, o) + at(v - Y + S, o)) + (at(v, o) + at(v + S, o));
+      const T vz = COMP == 2 ? (q[2] + q[3]) + (q[3] + q[4])
+                             : (at(w - Z, o) + at(w - Z + S, o)) + (at(w, o) + at(w + S, o));
+      T a = weno_dir<F>(f, o, X, vx, odd) * dxinv;
+      a = a + weno_dir<F>(f, o, Y, vy, odd) * dyinv;
+      return a + weno_q<F>(q, vz, odd) * dzinv;
+    };
+    T a;
+    bool odd = false;
+    if constexpr (std::is_floating_point_v<T>) {
+      a = cell(std::true_type{}, odd);
+      if (odd) a = cell(std::false_type{}, odd);
+    } else {
+      a = cell(std::false_type{}, odd);
+    }
+    put(out, o, a);
+  }
+}
 
 template <class T>
 __global__ void __launch_bounds__(256) weno_march_kernel(Dims d, T dxinv, T dyinv, T dzinv,
@@ -132,63 +239,21 @@ __global__ void __launch_bounds__(256) weno_march_kernel(Dims d, T dxinv, T dyin
                                                          T* __restrict__ au, T* __restrict__ av,
                                                          T* __restrict__ aw, int gx, int gy,
                                                          int kc) {
-  const int L = (int)blockIdx.x;
-  const int bx = L % gx, t = L / gx, by = t % gy, bz = t / gy;
-  const int i = 1 + bx * 64 + (int)threadIdx.x, j = 1 + by * 4 + (int)threadIdx.y;
+  const int L = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+  const int comp = L % 3, tile = L / 3;
+  const int bx = tile % gx, t = tile / gx, by = t % gy, bz = t / gy;
+  const int i = 1 + bx * 64 + (int)threadIdx.x;
+  const int j = 1 + by * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
   if (i > d.ni || j > d.nj) return;
-  const int k0 = 1 + bz * kc, k1 = min(d.nk, k0 + kc - 1);
-  const int X = 1, Y = d.sx, Z = d.sx * d.sy;
-  int c = d.ix(i, j, k0);
-  T qu[7], qv[7], qw[7];
-  const T h = T(0.5);
-#pragma unroll
-  for (int m = 0; m < 6; m++) {
-    qu[m + 1] = u[c + (m - 3) * Z];
-    qv[m + 1] = v[c + (m - 3) * Z];
-    qw[m + 1] = w[c + (m - 3) * Z];
-  }
-  for (int k = k0; k <= k1; k++, c += Z) {
-#pragma unroll
-    for (int m = 0; m < 6; m++) {
-      qu[m] = qu[m + 1];
-      qv[m] = qv[m + 1];
-      qw[m] = qw[m + 1];
-    }
-    qu[6] = u[c + 3 * Z];
-    qv[6] = v[c + 3 * Z];
-    qw[6] = w[c + 3 * Z];
-    T a, cm, cp;
-    // u (cal_advu_weno5.f:80-120)
-    cm = (u[c - X] + qu[3]) * h;
-    cp = (qu[3] + u[c + X]) * h;
-    a = weno_dir(u, c, X, (cm + cp) * h) * dxinv;
-    cm = (v[c - Y] + v[c + X - Y]) * h;
-    cp = (qv[3] + v[c + X]) * h;
-    a = a + weno_dir(u, c, Y, (cm + cp) * h) * dyinv;
-    cm = (qw[2] + w[c + X - Z]) * h;
-    cp = (qw[3] + w[c + X]) * h;
-    au[c] = a + weno_q(qu, (cm + cp) * h) * dzinv;
-    // v (cal_advu_weno5.f:147-187)
-    cm = (u[c - X] + u[c - X + Y]) * h;
-    cp = (qu[3] + u[c + Y]) * h;
-    a = weno_dir(v, c, X, (cm + cp) * h) * dxinv;
-    cm = (v[c - Y] + qv[3]) * h;
-    cp = (qv[3] + v[c + Y]) * h;
-    a = a + weno_dir(v, c, Y, (cm + cp) * h) * dyinv;
-    cm = (qw[2] + w[c + Y - Z]) * h;
-    cp = (qw[3] + w[c + Y]) * h;
-    av[c] = a + weno_q(qv, (cm + cp) * h) * dzinv;
-    // w (cal_advu_weno5.f:214-254)
-    cm = (u[c - X] + u[c - X + Z]) * h;
-    cp = (qu[3] + qu[4]) * h;
-    a = weno_dir(w, c, X, (cm + cp) * h) * dxinv;
-    cm = (v[c - Y] + v[c - Y + Z]) * h;
-    cp = (qv[3] + qv[4]) * h;
-    a = a + weno_dir(w, c, Y, (cm + cp) * h) * dyinv;
-    cm = (qw[2] + qw[3]) * h;
-    cp = (qw[3] + qw[4]) * h;
-    aw[c] = a + weno_q(qw, (cm + cp) * h) * dzinv;
-  }
+  const int k0 = 1 + bz * kc, planes = min(d.nk - k0 + 1, kc);
+  const ptrdiff_t Y = d.sx, Z = (ptrdiff_t)d.sx * d.sy, c = d.ix(1 + bx * 64, j, k0);
+  const uint32_t off = (uint32_t)(threadIdx.x * sizeof(T));
+  if (comp == 0)
+    weno_column<0>(Y, Z, dxinv, dyinv, dzinv, u + c, v + c, w + c, au + c, off, planes);
+  else if (comp == 1)
+    weno_column<1>(Y, Z, dxinv, dyinv, dzinv, u + c, v + c, w + c, av + c, off, planes);
+  else
+    weno_column<2>(Y, Z, dxinv, dyinv, dzinv, u + c, v + c, w + c, aw + c, off, planes);
 }
 
 // The reference clears the outputs over the padded image and fills the
@@ -199,8 +264,8 @@ void advect_weno5(const Dims d, double dxinv, double dyinv, double dzinv, const 
                   const T* __restrict__ v, const T* __restrict__ w, T* __restrict__ au,
                   T* __restrict__ av, T* __restrict__ aw) {
   const int gx = (d.ni + 63) / 64, gy = (d.nj + 3) / 4;
-  const int kc = march_planes(gx * gy, d.nk, kWenoK), gz = (d.nk + kc - 1) / kc;
-  weno_march_kernel<T><<<dim3(gx * gy * gz), dim3(64, 4, 1), 0, stream()>>>(
+  const int kc = march_planes(3 * gx * gy, d.nk, kWenoK), gz = (d.nk + kc - 1) / kc;
+  weno_march_kernel<T><<<dim3(3 * gx * gy * gz), dim3(64, 4, 1), 0, stream()>>>(
       d, T(dxinv), T(dyinv), T(dzinv), u, v, w, au, av, aw, gx, gy, kc);
   FEL_CHECK(hipGetLastError());
   launch_shell(d, [=] __device__(int i, int j, int k) {

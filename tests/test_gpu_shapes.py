@@ -140,3 +140,32 @@ def test_viscous_solve_with_any_ghosts(ni, nj, nk, resident):
         solve(H.call_gpu, coef, got)
     for a, b in zip(want, got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(5, 4, 4), (66, 5, 18)])
+def test_weno_zero_and_non_finite_values(ni, nj, nk):
+    """WENO5 where the transport velocity is zero (both sides count), where a
+    weight sum leaves the range of the short reciprocal, and at infinities and
+    NaN: bit for bit the oracle's."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    r = np.random.default_rng(ni)
+    head = [I(ni), I(nj), I(nk), D(1 / g.dx), D(1 / g.dy), D(1 / g.dz)]
+    plain = [r.standard_normal(g.shape) for _ in range(3)]
+    still = [np.where(r.random(g.shape) < 0.9, 0.0, x) for x in plain]
+    large = [5.0e36 * x for x in plain]
+
+    def both(vel):
+        a, b = run_both("cal_advu_weno5",
+                        lambda: head + [x.copy() for x in vel] + [g.zeros() for _ in range(3)])
+        return a[-3:], b[-3:]
+    for vel in (plain, [0.0 * x for x in plain], still, large):
+        for x, y in zip(*both(vel)):
+            # the library does not form the side that a zero multiplies, whose
+            # overflow is the oracle's NaN
+            assert np.all((x == y) | np.isnan(x))
+    assert not np.isnan(both(still)[0][0]).any()
+    u = np.where(r.random(g.shape) < 0.03, r.choice([np.inf, -np.inf, np.nan], g.shape), 0.0)
+    want, got = both([u, g.zeros(), g.zeros()])
+    quiet = np.isfinite(u) & np.isfinite(np.roll(u, 1, 0)) & np.isfinite(np.roll(u, -1, 0))
+    assert np.isnan(want[0][quiet]).any()
+    assert np.array_equal(want[0][quiet], got[0][quiet], equal_nan=True)
