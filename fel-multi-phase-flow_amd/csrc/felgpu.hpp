@@ -404,6 +404,23 @@ inline void launch_box(const Box& b, F f) {
   FEL_CHECK(hipGetLastError());
 }
 
+// Consecutive elements that a thread of a streaming kernel handles: 16 bytes, a
+// lane's widest access.  A run starts anywhere (the padded rows of the grid are
+// of any length): loads and stores of this width need only the element's own
+// alignment.
+template <class T>
+constexpr int kRun = sizeof(T) >= 16 ? 1 : 16 / (int)sizeof(T);
+
+template <int NV, class T>
+__device__ __forceinline__ void get_run(T* to, const T* from) {
+  __builtin_memcpy(to, from, NV * sizeof(T));
+}
+
+template <int NV, class T>
+__device__ __forceinline__ void put_run(T* to, const T* from) {
+  __builtin_memcpy(to, from, NV * sizeof(T));
+}
+
 // Planes per thread of a kernel that marches in k, gxy blocks per layer of
 // threads over nz planes: `most` where that leaves the chip full (2 blocks per
 // CU), fewer (`least` at the lowest) on smaller grids, whose time is one

@@ -169,3 +169,28 @@ def test_weno_zero_and_non_finite_values(ni, nj, nk):
     quiet = np.isfinite(u) & np.isfinite(np.roll(u, 1, 0)) & np.isfinite(np.roll(u, -1, 0))
     assert np.isnan(want[0][quiet]).any()
     assert np.array_equal(want[0][quiet], got[0][quiet], equal_nan=True)
+
+
+# rows of odd and even length, the image's end inside a 16-byte run (0 to 3
+# elements over), less than one block
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (5, 5, 5), (7, 5, 4), (33, 8, 10), (130, 9, 6)])
+def test_viscous_coefficients_on_the_image(ni, nj, nk):
+    """The 45 coefficient arrays over the whole padded image, in FP64 bit for
+    bit the oracle's, in FP32 within the rounding of their 4-point means and
+    products (fewer than 16 operations of 2^-24 each)."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    mu = np.random.default_rng(ni * nj * nk).uniform(0.1, 1.0, g.shape)
+    args = [I(ni), I(nj), I(nk), D(16.0), D(12.0), D(20.0)]
+    want, got = ([np.full(g.shape, 7.0) for _ in range(45)] for _ in range(2))
+    H.call_oracle("cal_arith_coef_vis", *args, mu, *want)
+    H.call_gpu("cal_arith_coef_vis", *args, mu, *got)
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
+    low = [np.full(g.shape, 7.0) for _ in range(45)]
+    H.gpu().felgpu_set_precision_(H.ctypes.byref(H.ctypes.c_int(32)))
+    try:
+        H.call_gpu("cal_arith_coef_vis", *args, mu, *low)
+    finally:
+        H.gpu().felgpu_set_precision_(H.ctypes.byref(H.ctypes.c_int(64)))
+    for a, b in zip(want, low):
+        assert np.max(np.abs(a - b)) <= 16 * 2.0 ** -24 * np.max(np.abs(a))
