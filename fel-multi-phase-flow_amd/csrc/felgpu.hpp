@@ -347,7 +347,6 @@ void deferred_chain_flush();
 void deferred_chain_check(const void* host, bool write);
 
 // Pinned host scratch for small device->host read-backs (reductions).
-double* pinned_scalars();  // 64 doubles
 void sync();
 
 // Device scratch reused across calls (grows, never shrinks).
@@ -649,8 +648,12 @@ using acc_t = std::conditional_t<is_f32<T>, double, T>;
 
 // Small device buffer for reduction results (slot-indexed, 16 doubles each).
 double* dev_scalars(int slot);
-// Copies n doubles from device to the pinned buffer and waits for them.
-const double* read_scalars(const double* dev, int n);
+// The same in pinned host memory, for results that the host reads: the last
+// kernel of a reduction writes them there itself, so that no copy (a launch,
+// 2 us and the gap before it) stands between it and the host.  await_scalars
+// waits for the stream and returns its argument.
+double* host_scalars(int slot);
+const double* await_scalars(const double* host);
 
 // Aborts with a message naming `who` unless the library runs in the FP64
 // mode (the adjoint routines have no FP32 or tangent form).

@@ -264,7 +264,7 @@ static void bndu_adj(const Dims d, double* u, double* v, double* w, double* wacc
 
 // Sum of the n values of a device array, added to *out on the host.
 void adjoint_add_sum(const double* a, int n, double* out) {
-  double* s = dev_scalars(21);
+  double* s = host_scalars(21);
   Dims p{};
   p.ni = n;
   p.nj = 1;
@@ -272,7 +272,7 @@ void adjoint_add_sum(const double* a, int n, double* out) {
   interior_reduce<1>(
       p, [=] __device__(int i, int, int, double* o) { o[0] = a[i - 1]; },
       [=] __device__(const double* t, double* o) { o[0] = t[0]; }, s);
-  *out += read_scalars(s, 1)[0];
+  *out += await_scalars(s)[0];
 }
 
 // ---------------------------------------------------------------------------

@@ -19,7 +19,7 @@ const double* vel_sums(const Dims d, const double* phi, const double* u, const d
   Call c("cal_vel_");
   const PT<T>* p = c.in_t<PT<T>>(phi, d.n3, "phi");
   const T *du = c.in_t<T>(u, d.n3, "u"), *dv = c.in_t<T>(v, d.n3, "v"), *dw = c.in_t<T>(w, d.n3, "w");
-  double* s = dev_scalars(7);
+  double* s = host_scalars(7);
   interior_reduce<4>(
       d,
       [=] __device__(int i, int j, int k, double* o) {
@@ -34,7 +34,7 @@ const double* vel_sums(const Dims d, const double* phi, const double* u, const d
         for (int m = 0; m < 4; m++) out[m] = t[m];
       },
       s);
-  const double* r = read_scalars(s, 4);
+  const double* r = await_scalars(s);
   c.finish();
   return r;
 }
@@ -87,12 +87,12 @@ double advmax_t(const Dims d, int jen, double dxinv, double dyinv, double dzinv,
   Call c("caldt_");
   const T *du = c.in_t<T>(u, d.n3, "u"), *dv = c.in_t<T>(v, d.n3, "v"), *dw = c.in_t<T>(w, d.n3, "w");
   double* part = static_cast<double*>(scratch(15, sizeof(double) * kRedBlocks));
-  double* out = dev_scalars(8);
+  double* out = host_scalars(8);
   advmax_stage1<T><<<kRedBlocks, 256, 0, stream()>>>(d, jen, dxinv, dyinv, dzinv, du, dv, dw, part);
   FEL_CHECK(hipGetLastError());
   advmax_stage2<<<1, 256, 0, stream()>>>(kRedBlocks, part, out);
   FEL_CHECK(hipGetLastError());
-  const double r = read_scalars(out, 1)[0];
+  const double r = await_scalars(out)[0];
   c.finish();
   return r;
 }
@@ -116,7 +116,7 @@ void cal_center_(const int* ipara, const int* ID, const int* svall, const int* n
   const double s1 = xl * 0.25, s2 = xl * 0.75;
   if (*area_pre1 == 1 && *area_pre2 == 3) *lap = *lap + 1;
   const int ap1 = *area_pre1, lp = *lap, id = *ID, njl = *nj;
-  double* s = dev_scalars(6);
+  double* s = host_scalars(6);
   const double* r = nullptr;
   with_flow([&](auto t) {
     using P = PT<decltype(t)>;
@@ -141,7 +141,7 @@ void cal_center_(const int* ipara, const int* ID, const int* svall, const int* n
           for (int m = 0; m < 4; m++) out[m] = t[m];
         },
         s);
-    r = read_scalars(s, 4);
+    r = await_scalars(s);
     c.finish();
   });
   center[0] = r[1] / r[0];

@@ -590,7 +590,7 @@ static void poisson_residual_pass(const Dims d, const double* div, const double*
 
 // |r| / |div| from the sums (0 when both vanish); waits for them.
 static double residual_ratio(const double* sums) {
-  const double* r = read_scalars(sums, 2);
+  const double* r = await_scalars(sums);
   if (r[0] > 0.0) return std::sqrt(r[1] / r[0]);
   return r[1] > 0.0 ? HUGE_VAL : 0.0;
 }
@@ -622,7 +622,7 @@ static void poisson_refine(const Dims d, double* dp, bool warm) {
   float* mr = static_cast<float*>(scratch(9, sizeof(float) * 2 * nm));
   float* mi = mr + nm;
   float* rc = residual_buffer(d);
-  double* sums = dev_scalars(9);
+  double* sums = host_scalars(9);
   // the right-hand side's current device copy (its buffer may have moved)
   Call c("solp_fft_tdma3_");
   const double* div = c.in_t<double>(pr.div_host, d.n3, "div");
@@ -651,9 +651,9 @@ void caldiv_t(const Dims d, double dxinv, double dyinv, double dzinv, double dt,
   const T *u = c.in_t<T>(uk, d.n3, "uk"), *v = c.in_t<T>(vk, d.n3, "vk"),
           *w = c.in_t<T>(wk, d.n3, "wk");
   PT<T>* dv = c.io_t<PT<T>>(div, d.n3, "div");
-  double* s = dev_scalars(3);
+  double* s = host_scalars(3);
   divergence<T>(d, dxinv, dyinv, dzinv, 1.0 / dt, u, v, w, dv, s);
-  *sum = read_scalars(s, 1)[0];
+  *sum = await_scalars(s)[0];
   c.finish();
 }
 
@@ -685,7 +685,7 @@ void tdma1_t(const Dims d, const double* div, double* phir_r, double* phir_i) {
     if (warm) {
       const double* dp0 = c.in_t<double>(rec.dp_host, d.n3, "dp");
       float* rc = residual_buffer(d);
-      poisson_residual_pass(d, dv, dp0, rc, dev_scalars(9));
+      poisson_residual_pass(d, dv, dp0, rc, host_scalars(9));
       fft_forward_of<T>(d, compact_rhs(d, rc), pr, pi);
     }
   }
@@ -745,11 +745,11 @@ template <class Q>
 double cal_av_t(const Dims d, const double* q) {
   Call c("cal_av_");
   const Q* dq = c.in_t<Q>(q, d.n3, "q");
-  double* s = dev_scalars(5);
+  double* s = host_scalars(5);
   interior_reduce<1>(
       d, [=] __device__(int i, int j, int k, double* o) { o[0] = val(dq[d.ix(i, j, k)]); },
       [=] __device__(const double* t, double* out) { out[0] = t[0]; }, s);
-  const double sum = read_scalars(s, 1)[0];
+  const double sum = await_scalars(s)[0];
   c.finish();
   return sum;
 }
@@ -1002,7 +1002,7 @@ void solp_fft_tdma4_(const int* ipara, const int* ID, const int* ndiv, const int
   (void)ipara;
   if (!(*imon_t > 0 && (*nstep % *imon_t) == 0)) return;
   const Dims d = make_dims(*ni, *nj, *nk);
-  double* s = dev_scalars(4);
+  double* s = host_scalars(4);
   const double* r = nullptr;
   with_flow([&](auto t) {
     using P = PT<decltype(t)>;
@@ -1010,7 +1010,7 @@ void solp_fft_tdma4_(const int* ipara, const int* ID, const int* ndiv, const int
     const P* dv = c.in_t<P>(div, d.n3, "div");
     const P* dd = c.in_t<P>(dp, d.n3, "dp");
     poisson_residual_sums<P>(d, *rho, *dxinv, *dyinv, *dzinv, dv, dd, s);
-    r = read_scalars(s, 2);
+    r = await_scalars(s);
     c.finish();
   });
   const double nn = (double)(*ni * *nj * *nk * *ndiv);
@@ -1027,7 +1027,7 @@ double felgpu_poisson_residual_(const int* ni, const int* nj, const int* nk, con
                                 const double* dxinv, const double* dyinv, const double* dzinv,
                                 const double* div, const double* dp) {
   const Dims d = make_dims(*ni, *nj, *nk);
-  double* s = dev_scalars(4);
+  double* s = host_scalars(4);
   const double* r = nullptr;
   with_flow([&](auto t) {
     using P = PT<decltype(t)>;
@@ -1035,7 +1035,7 @@ double felgpu_poisson_residual_(const int* ni, const int* nj, const int* nk, con
     const P* dv = c.in_t<P>(div, d.n3, "div");
     const P* dd = c.in_t<P>(dp, d.n3, "dp");
     poisson_residual_sums<P>(d, *rho, *dxinv, *dyinv, *dzinv, dv, dd, s);
-    r = read_scalars(s, 2);
+    r = await_scalars(s);
     c.finish();
   });
   const double nn = (double)(*ni * *nj * *nk);

@@ -362,7 +362,31 @@ struct PartSlots {
 
 // Two-stage fixed-order sum of the 12 launches' block partials: stage 1
 // reduces contiguous chunks (one block each), stage 2 the chunk sums.
-constexpr int kErrChunks = 256;
+// Up to kErrSerial partials a chunk, one launch does both: thread t adds chunk
+// t in registers, in stage 1's tree order (the sum of zeros padded to a power
+// of two), which saves a launch and its gap where a solve is launch-bound.
+constexpr int kErrChunks = 256, kErrSerial = 32;
+
+__global__ void __launch_bounds__(256) sor_err_small(const double* part, int n, double* out) {
+  __shared__ double sh[256];
+  const int t = (int)threadIdx.x;
+  const int per = (n + kErrChunks - 1) / kErrChunks;
+  const int b0 = t * per, b1 = min(n, b0 + per);
+  double v[kErrSerial];
+#pragma unroll
+  for (int m = 0; m < kErrSerial; m++) v[m] = b0 + m < b1 ? part[b0 + m] : 0.0;
+#pragma unroll
+  for (int s = kErrSerial / 2; s > 0; s >>= 1)
+#pragma unroll
+    for (int m = 0; m < s; m++) v[m] += v[m + s];
+  sh[t] = v[0];
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if (t < s) sh[t] += sh[t + s];
+    __syncthreads();
+  }
+  if (t == 0) out[0] = sh[0];
+}
 
 __global__ void __launch_bounds__(256) sor_err_stage1(const double* part, int n, double* chunk) {
   __shared__ double sh[256];
@@ -489,18 +513,17 @@ inline int sor_slot(const Dims& d) {
 }
 
 // Device work memory of one solve: the block partials of the 12 launches of
-// a sweep and their chunk sums (12 nb + kErrChunks doubles), the residual
-// sum (1 double) and the slip-wall coefficients (4 (ni+6)(nk+6) elements).
+// a sweep and their chunk sums (12 nb + kErrChunks doubles) and the slip-wall
+// coefficients (4 (ni+6)(nk+6) elements).
 template <class P>
 struct SorWork {
   double* part;
-  double* derr;
   P* wcoef;
 };
 
 template <class P>
 size_t sor_work_bytes(const Dims& d) {
-  const size_t a = sizeof(double) * ((size_t)sor_slot(d) * 12 + kErrChunks + 1);
+  const size_t a = sizeof(double) * ((size_t)sor_slot(d) * 12 + kErrChunks);
   const size_t wb = sizeof(P) * 4 * (size_t)d.sx * d.sz;
   return ((a + 255) / 256) * 256 + wb;
 }
@@ -508,10 +531,9 @@ size_t sor_work_bytes(const Dims& d) {
 // Lays the work memory out in one buffer of sor_work_bytes<P>(d) bytes.
 template <class P>
 SorWork<P> sor_work_in(const Dims& d, void* buf) {
-  const size_t a = sizeof(double) * ((size_t)sor_slot(d) * 12 + kErrChunks + 1);
+  const size_t a = sizeof(double) * ((size_t)sor_slot(d) * 12 + kErrChunks);
   SorWork<P> w;
   w.part = static_cast<double*>(buf);
-  w.derr = w.part + (size_t)sor_slot(d) * 12 + kErrChunks;
   w.wcoef = reinterpret_cast<P*>(static_cast<char*>(buf) + ((a + 255) / 256) * 256);
   return w;
 }
@@ -537,7 +559,7 @@ SorResult sor4(const Dims d, SorArgs<T> a, bool onfly, bool lo, bool hi, double 
     const int n = 12 * slotn;
     launch_flat(n, [=] __device__(int m) { part[m] = 0.0; });
   }
-  double* derr = work.derr;
+  double* err2 = host_scalars(10);
   // in-launch ghost refresh needs even ni, nk (colour parity of periodic images)
   const bool fuse_ok = d.ni % 2 == 0 && d.nk % 2 == 0;
   // pairs 1 and 2 in one launch (with the per-solve face-density table)
@@ -631,10 +653,14 @@ SorResult sor4(const Dims d, SorArgs<T> a, bool onfly, bool lo, bool hi, double 
         }
       }
     }
-    sor_err_stage1<<<kErrChunks, 256, 0, stream()>>>(part, 12 * slotn, chunk);
-    sor_err_stage2<<<1, 256, 0, stream()>>>(chunk, derr);
+    if (12 * slotn <= kErrChunks * kErrSerial) {
+      sor_err_small<<<1, 256, 0, stream()>>>(part, 12 * slotn, err2);
+    } else {
+      sor_err_stage1<<<kErrChunks, 256, 0, stream()>>>(part, 12 * slotn, chunk);
+      sor_err_stage2<<<1, 256, 0, stream()>>>(chunk, err2);
+    }
     FEL_CHECK(hipGetLastError());
-    const double sum = read_scalars(derr, 1)[0];
+    const double sum = await_scalars(err2)[0];
     err = std::sqrt(sum / (double)(d.ni * d.nj * d.nk * ndiv)) + 1.0e-99;
     if (lp == 0) err0 = err;
     if (err / err0 <= 1.0e-3) break;

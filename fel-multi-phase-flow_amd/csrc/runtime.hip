@@ -247,7 +247,7 @@ void ensure_init() {
   FEL_CHECK(hipSetDevice(r.device));
   sor_noalloc_setup();
   FEL_CHECK(hipStreamCreateWithFlags(&r.s, hipStreamNonBlocking));
-  FEL_CHECK(hipHostMalloc((void**)&r.pinned, 64 * sizeof(double), hipHostMallocDefault));
+  FEL_CHECK(hipHostMalloc((void**)&r.pinned, 64 * 16 * sizeof(double), hipHostMallocDefault));
   FEL_CHECK(hipMalloc((void**)&r.dscal, 64 * 16 * sizeof(double)));
   FEL_CHECK(hipMemsetAsync(r.dscal, 0, 64 * 16 * sizeof(double), r.s));
   const char* pr = std::getenv("FELGPU_PRECISION");
@@ -374,9 +374,9 @@ void* scratch(int slot, size_t bytes) {
   return r.scratch_ptr[slot];
 }
 
-double* pinned_scalars() {
+double* host_scalars(int slot) {
   ensure_init();
-  return R().pinned;
+  return R().pinned + 16 * slot;
 }
 
 double* dev_scalars(int slot) {
@@ -412,11 +412,9 @@ char* fortran_e(char* out, double v, int w, int d) {
   return out;
 }
 
-const double* read_scalars(const double* dev, int n) {
-  Runtime& r = R();
-  FEL_CHECK(hipMemcpyAsync(r.pinned, dev, sizeof(double) * n, hipMemcpyDeviceToHost, r.s));
-  FEL_CHECK(hipStreamSynchronize(r.s));
-  return r.pinned;
+const double* await_scalars(const double* host) {
+  FEL_CHECK(hipStreamSynchronize(R().s));
+  return host;
 }
 
 // --------------------------------------------------------------------------

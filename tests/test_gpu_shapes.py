@@ -107,8 +107,10 @@ def test_marching_stencils_shapes(ni, nj, nk):
 
 
 # even x and z (ghost images in the launches: the smallest grid, one and several
-# blocks a row) and an odd size of each (refresh launches)
-@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (66, 7, 18), (130, 9, 6), (33, 8, 10), (8, 5, 9)])
+# blocks a row) and an odd size of each (refresh launches); partial sums of the
+# stop test for one launch and for two
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (66, 7, 18), (130, 9, 6), (33, 8, 10), (8, 5, 9),
+                                      (8, 8, 340), (8, 8, 1400)])
 @pytest.mark.parametrize("resident", [False, True], ids=["coefficients", "viscosity"])
 def test_viscous_solve_with_any_ghosts(ni, nj, nk, resident):
     """solu_sor4 from ghosts that are no periodic images: the values that its
