@@ -58,23 +58,68 @@ __device__ __forceinline__ void take(double* q, int g, int s) {
   q[g] = 0.0;
 }
 
+// The transposed ghost fills of one line of n cells (elements -2..n+3, `st`
+// apart, q pointing at element -2).  Plain: the six periodic ghosts.  Shifted:
+// bndu's u in x and w in z, whose ghosts -2..0 are copies of n-1..n+1 and which
+// leaves n+1 as it is.  The twelve elements at the two ends are read together,
+// folded in registers and written together: element by element, each sum waits
+// for the store before it (15 such steps one after the other: bndu_adj's
+// launches 11.7 us at 128x64x128, this form 8.4; periodic_adj's 5.5 and 4.6).  Lines of fewer than 6 cells, whose ends share
+// elements, are folded element by element.
+struct LineEnds {
+  double a[12];  // elements -2..3, then n-2..n+3
+  __device__ __forceinline__ LineEnds(const double* q, int st, int n) {
+#pragma unroll
+    for (int m = 0; m < 6; m++) {
+      a[m] = q[m * st];
+      a[6 + m] = q[(n + m) * st];
+    }
+  }
+  __device__ __forceinline__ void fold(int g, int s) {
+    a[s] = a[s] + a[g];
+    a[g] = 0.0;
+  }
+  template <bool SHIFTED>
+  __device__ __forceinline__ void fold_all() {
+    fold(11, 5);
+    fold(10, 4);
+    if (!SHIFTED) fold(9, 3);
+    fold(0, SHIFTED ? 7 : 6);
+    fold(1, SHIFTED ? 8 : 7);
+    fold(2, SHIFTED ? 9 : 8);
+  }
+  __device__ __forceinline__ void store(double* q, int st, int n) const {
+#pragma unroll
+    for (int m = 0; m < 6; m++) {
+      q[m * st] = a[m];
+      q[(n + m) * st] = a[6 + m];
+    }
+  }
+};
+constexpr int kMinEnds = 6;
+
+template <bool SHIFTED>
+__device__ __forceinline__ void fold_line(double* q, int st, int n) {
+  const int sh = SHIFTED ? 1 : 0;
+  for (int g = 3; g > sh; g--) take(q, (n + g + 2) * st, (g + 2) * st);
+  for (int g = -2; g <= 0; g++) take(q, (g + 2) * st, (n + g + sh + 2) * st);
+}
+
 // srcs/bnd_periodic.f:14-43 transposed: the z pass (every (i,j) line), then
 // the x pass (every (j,k) line), each in reverse.
 static void periodic_adj(const Dims d, double* q) {
-  const int ni = d.ni, nk = d.nk, sx = d.sx, sy = d.sy, sz = d.sz, Z = d.sx * d.sy;
-  launch_flat(sx * sy, [=] __device__(int m) {
-    const int c = m;  // (i, j, k = -2) is m + 0 * Z
-    const int g[6] = {0, 1, 2, nk + 3, nk + 4, nk + 5};   // k = -2..0, nk+1..nk+3
-    const int s[6] = {nk, nk + 1, nk + 2, 3, 4, 5};       // k = nk-2..nk, 1..3
-    for (int t = 5; t >= 0; t--) take(q, c + g[t] * Z, c + s[t] * Z);
-  });
-  launch_flat(sy * sz, [=] __device__(int m) {
-    const int c = m * sx;  // (i = -2, j, k)
-    const int g[6] = {0, 1, 2, ni + 3, ni + 4, ni + 5};
-    const int s[6] = {ni, ni + 1, ni + 2, 3, 4, 5};
-    for (int t = 5; t >= 0; t--) take(q, c + g[t], c + s[t]);
-  });
-  (void)sz;
+  const int sx = d.sx, sy = d.sy, Z = d.sx * d.sy;
+  auto line = [=] __device__(double* p, int st, int n) {
+    if (n >= kMinEnds) {
+      LineEnds e(p, st, n);
+      e.fold_all<false>();
+      e.store(p, st, n);
+    } else {
+      fold_line<false>(p, st, n);
+    }
+  };
+  launch_flat(sx * sy, [=] __device__(int m) { line(q + m, Z, d.nk); });
+  launch_flat(sy * d.sz, [=] __device__(int m) { line(q + m * sx, 1, d.ni); });
 }
 
 // srcs/bnd_neumann.f:14-41 transposed (mirror ghosts of the j walls).
@@ -92,13 +137,14 @@ static void neumann_adj(const Dims d, double* q, bool lo, bool hi) {
 }
 
 // Parameter adjoints of bndu (bndu_bp_): the call's input velocities on
-// the rows next to the walls (rows: u at j = 1, u at j = nj, w at j = 1, w
-// at j = nj, one value per (i,k) column each), uwall, and the adjoints of
+// the rows next to the walls (u1: u at j = 1, un: u at j = nj, w1, wn: w, each
+// at column (-2,-2); the next k is rowk elements on), uwall, and the adjoints of
 // the slip lengths and phi; pa holds the phi_av adjoint of each wall cell
 // (bottom then top, one value per (i,k) column).  l1b == nullptr: none
 // formed.
 struct BnduParam {
-  const double* rows;
+  const double *u1, *un, *w1, *wn;
+  int rowk;
   double uwall;
   double *l1b, *l2b, *phib, *pa;
 };
@@ -154,107 +200,129 @@ static void bndu_phi_gather(const Dims d, const BnduParam bp, bool lo, bool hi) 
 // beyond folded in), gives c1_b = A (-+uwall) and c2_b = A_u u1 + A_w w1.
 static void bndu_adj(const Dims d, double* u, double* v, double* w, double* wacc, double dy,
                      const double* l1, const double* l2, const double* phi, bool lo, bool hi,
-                     const BnduParam bp = BnduParam{nullptr, 0.0, nullptr, nullptr, nullptr,
-                                                    nullptr}) {
-  const int ni = d.ni, nj = d.nj, nk = d.nk, sx = d.sx, sy = d.sy, Z = d.sx * d.sy;
-  // z fills (bndu.f:130-155), every (i,j) line, statements reversed
-  launch_flat(sx * sy, [=] __device__(int c) {
-    auto kz = [=](int k) { return c + (k + 2) * Z; };
-    take(w, kz(nk + 3), kz(3)); take(w, kz(nk + 2), kz(2));
-    take(v, kz(nk + 3), kz(3)); take(v, kz(nk + 2), kz(2)); take(v, kz(nk + 1), kz(1));
-    take(u, kz(nk + 3), kz(3)); take(u, kz(nk + 2), kz(2)); take(u, kz(nk + 1), kz(1));
-    take(w, kz(-2), kz(nk - 1)); take(w, kz(-1), kz(nk)); take(w, kz(0), kz(nk + 1));
-    take(v, kz(-2), kz(nk - 2)); take(v, kz(-1), kz(nk - 1)); take(v, kz(0), kz(nk));
-    take(u, kz(-2), kz(nk - 2)); take(u, kz(-1), kz(nk - 1)); take(u, kz(0), kz(nk));
+                     const BnduParam bp = BnduParam{}) {
+  const int nj = d.nj, sx = d.sx, sy = d.sy, Z = d.sx * d.sy;
+  // z fills (bndu.f:130-155), every (i,j) line
+  launch_flat(sx * sy, [=] __device__(int m) {
+    const int n = d.nk;
+    if (n >= kMinEnds) {
+      LineEnds eu(u + m, Z, n), ev(v + m, Z, n), ew(w + m, Z, n);
+      eu.fold_all<false>();
+      ev.fold_all<false>();
+      ew.fold_all<true>();
+      eu.store(u + m, Z, n);
+      ev.store(v + m, Z, n);
+      ew.store(w + m, Z, n);
+    } else {
+      fold_line<false>(u + m, Z, n);
+      fold_line<false>(v + m, Z, n);
+      fold_line<true>(w + m, Z, n);
+    }
   });
-  // x fills (bndu.f:104-127), every (j,k) line, statements reversed
+  // x fills (bndu.f:104-127), every (j,k) line
   launch_flat(sy * d.sz, [=] __device__(int m) {
-    const int c = m * sx;
-    auto ix = [=](int i) { return c + i + 2; };
-    take(w, ix(ni + 3), ix(3)); take(w, ix(ni + 2), ix(2)); take(w, ix(ni + 1), ix(1));
-    take(v, ix(ni + 3), ix(3)); take(v, ix(ni + 2), ix(2)); take(v, ix(ni + 1), ix(1));
-    take(u, ix(ni + 3), ix(3)); take(u, ix(ni + 2), ix(2));
-    take(w, ix(-2), ix(ni - 2)); take(w, ix(-1), ix(ni - 1)); take(w, ix(0), ix(ni));
-    take(v, ix(-2), ix(ni - 2)); take(v, ix(-1), ix(ni - 1)); take(v, ix(0), ix(ni));
-    take(u, ix(-2), ix(ni - 1)); take(u, ix(-1), ix(ni)); take(u, ix(0), ix(ni + 1));
+    const int n = d.ni, c = m * sx;
+    if (n >= kMinEnds) {
+      LineEnds eu(u + c, 1, n), ev(v + c, 1, n), ew(w + c, 1, n);
+      eu.fold_all<true>();
+      ev.fold_all<false>();
+      ew.fold_all<false>();
+      eu.store(u + c, 1, n);
+      ev.store(v + c, 1, n);
+      ew.store(w + c, 1, n);
+    } else {
+      fold_line<true>(u + c, 1, n);
+      fold_line<false>(v + c, 1, n);
+      fold_line<false>(w + c, 1, n);
+    }
   });
   if (!lo && !hi) return;
   const int nw = sx * d.sz;
-  // wall rows (bndu.f:29-98), every (i,k) column, top wall first
+  // wall rows (bndu.f:29-98), every (i,k) column, top wall first; the rows of
+  // u and w (q: w, u) from the wall's first row outwards are read together
   launch_flat(nw, [=] __device__(int m) {
-    const int i = m % sx - 2, k = m / sx - 2;
+    const int i = m % sx - 2, k = m / sx - 2, rm = m % sx + m / sx * bp.rowk;
     auto jy = [=](int j) { return d.ix(i, j, k); };
     double acc = 0.0;
+    double* qs[2] = {w, u};
+    double top[2][4], bot[2][4];
+    WallCoef<double> ct{}, cb{};
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        top[t][g] = hi ? qs[t][jy(nj + g)] : 0.0;
+        bot[t][g] = lo ? qs[t][jy(1 - g)] : 0.0;
+      }
+    if (hi) ct = wall_coef(d, i, nj, k, dy, l1, l2, phi);
+    if (lo) cb = wall_coef(d, i, 1, k, dy, l1, l2, phi);
+    // g1 = c1 (-+uwall) + c2 q; g2 = 2 g1 - q; g3 = 2 g2 - g1, reversed: the
+    // adjoint of g1, with that of q (r[0]) completed
+    auto rows_adj = [](double* r, double c2) {
+      r[2] = r[2] + 2.0 * r[3];
+      r[1] = r[1] - r[3];
+      r[1] = r[1] + 2.0 * r[2];
+      r[0] = r[0] - r[2];
+      r[0] = r[0] + c2 * r[1];
+      return r[1];
+    };
     if (hi) {
-      const WallCoef<double> cf = wall_coef(d, i, nj, k, dy, l1, l2, phi);
       double c1b = 0.0, c2b = 0.0;
-      // u, w: g1 = c1 (+uwall) + c2 q(nj); g2 = 2 g1 - q(nj); g3 = 2 g2 - g1
-      double* qs[2] = {w, u};
+#pragma unroll
       for (int t = 0; t < 2; t++) {
-        double* q = qs[t];
-        const double b3 = q[jy(nj + 3)];
-        q[jy(nj + 2)] = q[jy(nj + 2)] + 2.0 * b3;
-        q[jy(nj + 1)] = q[jy(nj + 1)] - b3;
-        q[jy(nj + 3)] = 0.0;
-        const double b2 = q[jy(nj + 2)];
-        q[jy(nj + 1)] = q[jy(nj + 1)] + 2.0 * b2;
-        q[jy(nj)] = q[jy(nj)] - b2;
-        q[jy(nj + 2)] = 0.0;
-        const double b1 = q[jy(nj + 1)];
-        q[jy(nj)] = q[jy(nj)] + cf.c2 * b1;
-        if (t == 1) acc = acc + cf.c1 * b1;
+        const double b1 = rows_adj(top[t], ct.c2);
+        if (t == 1) acc = acc + ct.c1 * b1;
         if (bp.l1b) {
           if (t == 0) {
-            c2b = c2b + b1 * bp.rows[3 * nw + m];
+            c2b = c2b + b1 * bp.wn[rm];
           } else {
             c1b = c1b + b1 * bp.uwall;
-            c2b = c2b + b1 * bp.rows[nw + m];
+            c2b = c2b + b1 * bp.un[rm];
           }
         }
-        q[jy(nj + 1)] = 0.0;
+        qs[t][jy(nj)] = top[t][0];
+        for (int g = 1; g <= 3; g++) qs[t][jy(nj + g)] = 0.0;
       }
       if (bp.l1b)
         bp.pa[m + nw] = wall_coef_b(d, i, nj, k, dy, l1, l2, phi, c1b, c2b, bp.l1b, bp.l2b);
       // v: v(nj) = 0, v(nj+g) = -v(nj-g)
-      for (int g = 3; g >= 1; g--) {
-        v[jy(nj - g)] = v[jy(nj - g)] - v[jy(nj + g)];
-        v[jy(nj + g)] = 0.0;
+      double in[3], gh[3];
+#pragma unroll
+      for (int g = 0; g < 3; g++) {
+        in[g] = v[jy(nj - 1 - g)];
+        gh[g] = v[jy(nj + 1 + g)];
+      }
+#pragma unroll
+      for (int g = 0; g < 3; g++) {
+        v[jy(nj - 1 - g)] = in[g] - gh[g];
+        v[jy(nj + 1 + g)] = 0.0;
       }
       v[jy(nj)] = 0.0;
     }
     if (lo) {
-      const WallCoef<double> cf = wall_coef(d, i, 1, k, dy, l1, l2, phi);
       double c1b = 0.0, c2b = 0.0;
-      double* qs[2] = {w, u};
+#pragma unroll
       for (int t = 0; t < 2; t++) {
-        double* q = qs[t];
-        const double b3 = q[jy(-2)];
-        q[jy(-1)] = q[jy(-1)] + 2.0 * b3;
-        q[jy(0)] = q[jy(0)] - b3;
-        q[jy(-2)] = 0.0;
-        const double b2 = q[jy(-1)];
-        q[jy(0)] = q[jy(0)] + 2.0 * b2;
-        q[jy(1)] = q[jy(1)] - b2;
-        q[jy(-1)] = 0.0;
-        const double b1 = q[jy(0)];
-        q[jy(1)] = q[jy(1)] + cf.c2 * b1;
-        if (t == 1) acc = acc - cf.c1 * b1;
+        const double b1 = rows_adj(bot[t], cb.c2);
+        if (t == 1) acc = acc - cb.c1 * b1;
         if (bp.l1b) {
           if (t == 0) {
-            c2b = c2b + b1 * bp.rows[2 * nw + m];
+            c2b = c2b + b1 * bp.w1[rm];
           } else {
             c1b = c1b - b1 * bp.uwall;
-            c2b = c2b + b1 * bp.rows[m];
+            c2b = c2b + b1 * bp.u1[rm];
           }
         }
-        q[jy(0)] = 0.0;
+        qs[t][jy(1)] = bot[t][0];
+        for (int g = 1; g <= 3; g++) qs[t][jy(1 - g)] = 0.0;
       }
       if (bp.l1b) bp.pa[m] = wall_coef_b(d, i, 1, k, dy, l1, l2, phi, c1b, c2b, bp.l1b, bp.l2b);
       // v: v(-2) = -v(2), v(-1) = -v(1), v(0) = 0
+      const double i1 = v[jy(1)], i2 = v[jy(2)], g1 = v[jy(-1)], g2 = v[jy(-2)];
       v[jy(0)] = 0.0;
-      v[jy(1)] = v[jy(1)] - v[jy(-1)];
+      v[jy(1)] = i1 - g1;
       v[jy(-1)] = 0.0;
-      v[jy(2)] = v[jy(2)] - v[jy(-2)];
+      v[jy(2)] = i2 - g2;
       v[jy(-2)] = 0.0;
     }
     if (wacc) wacc[m] = wacc[m] + acc;
@@ -920,7 +988,7 @@ static void for_pair_cells(const Dims d, int jen, int p, F f) {
 }
 
 // The rows next to the walls of u and w (j = 1 and j = nj, every (i,k)
-// column) into rows[4 nw], the layout BnduParam reads.
+// column) into rows[4 nw].
 static void wall_rows(const Dims d, const double* u, const double* w, double* rows) {
   const int nj = d.nj, sx = d.sx, nw = d.sx * d.sz;
   launch_flat(nw, [=] __device__(int m) {
@@ -1457,8 +1525,13 @@ static void sor_bp_run(const Dims d, const int* nID, SorAdj& a, SorParam& sp, Bn
   double* work = static_cast<double*>(scratch(42, sizeof(double) * (3 * n3 + slot * 12 * (size_t)nsw)));
   double* X[3] = {work, work + n3, work + 2 * n3};
   double* undo = work + 3 * n3;
-  double* rows = static_cast<double*>(scratch(45, sizeof(double) * 4 * nw));
-  bp.rows = rows;
+  // the rows next to the walls, read where the state stands
+  const int row1 = d.ix(-2, 1, -2), rown = d.ix(-2, d.nj, -2);
+  bp.u1 = X[0] + row1;
+  bp.un = X[0] + rown;
+  bp.w1 = X[2] + row1;
+  bp.wn = X[2] + rown;
+  bp.rowk = d.sx * d.sy;
   const double uw = uwall, dyv = dy;
   const int jen = a.jen;
   for (int r = 0; r < 3; r++) copy_dev(X[r], x0[r], d.n3);
@@ -1478,7 +1551,6 @@ static void sor_bp_run(const Dims d, const int* nID, SorAdj& a, SorParam& sp, Bn
         double* u = undo + slot * (size_t)((s * 3 + q) * 4 + p);
         // X: the state before the refresh, then before the pair
         shell_restore(shell, ns, X, u + np);
-        wall_rows(d, X[0], X[2], rows);
         periodic_adj(d, a.lb[q]);
         bndu_adj(d, a.lb[0], a.lb[1], a.lb[2], wacc, dyv, dl1, dl2, dphi, lo, hi, bp);
         const int is = kIsor[2 * p], js = kJsor[2 * p], ks = kKsor[2 * p];
@@ -1811,7 +1883,11 @@ void bndu_bp_(const int* nID, const int* ni, const int* nj, const int* nk, const
   BnduParam bp;
   double* rows = static_cast<double*>(scratch(45, sizeof(double) * 4 * nw));
   wall_rows(d, c.in(uk, d.n3, "uk"), c.in(wk, d.n3, "wk"), rows);
-  bp.rows = rows;
+  bp.u1 = rows;
+  bp.un = rows + nw;
+  bp.w1 = rows + 2 * nw;
+  bp.wn = rows + 3 * nw;
+  bp.rowk = d.sx;
   bp.uwall = *uwall;
   double* ub = c.io(ukb, d.n3, "ukb");
   double* vb = c.io(vkb, d.n3, "vkb");

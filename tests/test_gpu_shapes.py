@@ -4,6 +4,7 @@ a shape changes."""
 import numpy as np
 import pytest
 
+import adjoint_cases as A
 import felharness as H
 from felharness import D, I, Grid
 from test_gpu_kernels import check, grad, run_both
@@ -196,3 +197,19 @@ def test_viscous_coefficients_on_the_image(ni, nj, nk):
         H.gpu().felgpu_set_precision_(H.ctypes.byref(H.ctypes.c_int(64)))
     for a, b in zip(want, low):
         assert np.max(np.abs(a - b)) <= 16 * 2.0 ** -24 * np.max(np.abs(a))
+
+
+# lines of 4 and 5 cells (ends that share elements) and of 6 and 7 (the first
+# whose two ends are folded in registers) in x and z, the shortest columns in y
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (5, 4, 6), (6, 5, 5), (7, 6, 4), (6, 4, 7)])
+@pytest.mark.parametrize("case", ["bndu", "bndu_bp", "bnd_periodic"])
+def test_ghost_adjoints_on_short_lines(ni, nj, nk, case):
+    """The transposed ghost fills and wall rows equal the oracle's, to the
+    rounding of the slip coefficients' adjoints."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    c = {"bndu": A.Bndu, "bndu_bp": A.BnduP, "bnd_periodic": A.Periodic}[case](g, ni + 7 * nk)
+    x, y = c.inputs(), c.out_adjoints()
+    want = c.adjoint(H.call_oracle, {k: v.copy() for k, v in y.items()})
+    got = c.adjoint(H.call_gpu, {k: v.copy() for k, v in y.items()})
+    for k in x:
+        assert np.max(np.abs(want[k] - got[k])) <= 1e-13 * max(1.0, np.max(np.abs(want[k])))
