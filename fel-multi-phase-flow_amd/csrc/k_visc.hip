@@ -40,14 +40,8 @@ void calphat(const Dims d, const T* p, const T* po, T* phat) {
 template <class T>
 void grad_faces(const Dims d, double dxinv_, double dyinv_, double dzinv_, const T* q, T* qx, T* qy,
                 T* qz) {
-  const T dxinv = T(dxinv_), dyinv = T(dyinv_), dzinv = T(dzinv_);
-  launch_box(Box{-2, d.ni + 2, -2, d.nj + 2, -2, d.nk + 2}, [=] __device__(int i, int j, int k) {
-    const int c = d.ix(i, j, k);
-    const T q0 = q[c];
-    qx[c] = (-q0 + q[c + 1]) * dxinv;
-    qy[c] = (-q0 + q[c + d.sx]) * dyinv;
-    qz[c] = (-q0 + q[c + d.sx * d.sy]) * dzinv;
-  });
+  const T dyinv = T(dyinv_);
+  forward_differences(d, T(dxinv_), [=] __device__(int) { return dyinv; }, T(dzinv_), q, qx, qy, qz);
 }
 
 // srcs/calsij.f:28-139

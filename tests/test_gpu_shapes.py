@@ -213,3 +213,22 @@ def test_ghost_adjoints_on_short_lines(ni, nj, nk, case):
     got = c.adjoint(H.call_gpu, {k: v.copy() for k, v in y.items()})
     for k in x:
         assert np.max(np.abs(want[k] - got[k])) <= 1e-13 * max(1.0, np.max(np.abs(want[k])))
+
+
+# rows of even and odd length, the image's last run whole or cut
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (5, 5, 5), (7, 4, 6), (33, 8, 10), (130, 9, 6)])
+def test_streamed_differences_shapes(ni, nj, nk):
+    """Face gradients (one 1/dy and one per row) and the surface force by 16-byte
+    runs: bit for bit the oracle's, with the elements they leave untouched."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    r = np.random.default_rng(ni + nj + nk)
+    f = [r.standard_normal(g.shape) for _ in range(10)]
+    rk = r.standard_normal((3,) + g.shape)
+    scales = [D(16.0), D(12.0), D(20.0)]
+    for dy in (np.full(nj + 6, 12.0), r.uniform(8.0, 16.0, nj + 6)):
+        check(*run_both("cal_grad_p2uvw", lambda: [
+            I(0), I(nj), I(ni), I(nj), I(nk), scales[0], dy, scales[2]] + [x.copy() for x in f[:4]]))
+    check(*run_both("cal_grad_prs", lambda: [I(ni), I(nj), I(nk)] + scales +
+                    [x.copy() for x in f[:4]]))
+    check(*run_both("calfst", lambda: [I(ni), I(nj), I(nk), D(0.81), D(8.1e-4), D(5.5)] +
+                    [x.copy() for x in f[4:7]] + [rk.copy()] + [x.copy() for x in f[7:10]]))
