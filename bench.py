@@ -30,7 +30,7 @@ stream inside the timed region.  The launches go through
 hipExtLaunchKernelGGL, which stamps an event with its own launch's start or
 end, so the timing adds no packets between launches: the three pairs of a
 sweep that run back to back are one timed span (start of the first to the
-end of the third, divided by three), the pair before a ghost-refresh launch
+end of the third, divided by three), the first pair of each sweep
 is not timed.  The CPU
 baseline is the reference's own program (srcs/main.f90 and its makefile
 sources, built with OpenMP by oracle/ref_main.py) timed on this host's cores

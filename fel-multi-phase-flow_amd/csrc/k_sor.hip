@@ -626,7 +626,7 @@ SorResult sor4(const Dims d, SorArgs<T> a, bool onfly, bool lo, bool hi, double 
                          : (p == 0 ? kFirst : kLater);
         const int nt = xcd_arg(1, nb);
         // The colour-pair timer: with pairs 1 and 2 joined, pair 3 (pair 0
-        // is followed by a refresh launch and not timed); with fused images
+        // of the solve is followed by a refresh launch); with fused images
         // only, pairs 1-3 back to back as one span of three launches;
         // without them every pair is a span of its own.
         hipEvent_t e0 = nullptr, e1 = nullptr;
