@@ -231,31 +231,42 @@ __device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c,
 }
 
 // FORM != kStored: the pair's ghost images are written by the launch.
+// Bound by memory (512x128x256, FP64: 132-144 us a launch).  A wavefront is one
+// row of 64 cells, and its row index is made scalar, so the rows' addresses
+// stay out of the vector registers: 62-68 of them (7-8 wavefronts a SIMD) with
+// nothing spilled, which the allocation-free solve needs (private memory is
+// backed by device memory on demand).  With the row in vector registers and
+// their number bounded to 64, the forms that read shifted ghosts spilled: w's
+// pair 0 and pair 3 took 149 and 143 us, now 144 and 138; v's 143 and 135, now
+// 140 and 134.  The forms that read coefficient arrays and shifted ghosts went
+// from 76-90 to 64-66 registers, the tangent mode's from 74-118 to 66-94, their
+// times unchanged (300-305 us; 17-19 us at 128x64x128).
 template <int COMP, bool ONFLY, int FORM, class T, bool R00I = false>
-__global__ void __launch_bounds__(512, ONFLY && sizeof(T) == 8 ? 8 : 1) sor_pair_kernel(Dims d, SorArgs<T> a, int is, int js, int ks,
+__global__ void __launch_bounds__(512) sor_pair_kernel(Dims d, SorArgs<T> a, int is, int js, int ks,
                                                        int jend, int gx, int gy, int ntiles,
                                                        double* part) {
   const int L = xcd_tile((int)blockIdx.x, ntiles);
   const int bx = L % gx, tt = L / gx, by = tt % gy, bz = tt / gy;
   double e = 0.0;
   for (int kz = 0; kz < kKB; kz++) {
-  const int k = 1 + bz * kKB + kz;
-  if (k > d.nk) break;
-  const int q = (k - ks) & 1;
-  const int ii = bx * 64 + (int)threadIdx.x;
-  const int i = 1 + ((is + q - 1) & 1) + 2 * ii;
-  const int j = 1 + ((js + q - 1) & 1) + 2 * (by * (int)blockDim.y + (int)threadIdx.y);
-  if (i <= d.ni && j <= jend) {
-    const int X = 1;
-    const int c = d.ix(i, j, k);
-    const int ridx = r00_index(d, ii, by * (int)blockDim.y + (int)threadIdx.y, k);
-    T* F = COMP == 0 ? a.un : (COMP == 1 ? a.vn : a.wn);
-    // u's own ghost column 0 before its first pair: u(ni+1)
-    const T xm = F[COMP == 0 && FORM == kFirst && i == 1 ? c + d.ni : c - X];
-    const T nv = sor_cell<COMP, ONFLY, FORM, T, R00I>(d, a, c, i, k, ridx, xm, F[c + X], e);
-    put_update(F, c, nv);
-    if (FORM != kStored) write_images<COMP>(d, a, F, i, j, k, nv);
-  }
+    const int k = 1 + bz * kKB + kz;
+    if (k > d.nk) break;
+    const int q = (k - ks) & 1;
+    const int ii = bx * 64 + (int)threadIdx.x;
+    const int jj = by * (int)blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int i = 1 + ((is + q - 1) & 1) + 2 * ii;
+    const int j = 1 + ((js + q - 1) & 1) + 2 * jj;
+    if (i <= d.ni && j <= jend) {
+      const int X = 1;
+      const int c = d.ix(i, j, k);
+      const int ridx = r00_index(d, ii, jj, k);
+      T* F = COMP == 0 ? a.un : (COMP == 1 ? a.vn : a.wn);
+      // u's own ghost column 0 before its first pair: u(ni+1)
+      const T xm = F[COMP == 0 && FORM == kFirst && i == 1 ? c + d.ni : c - X];
+      const T nv = sor_cell<COMP, ONFLY, FORM, T, R00I>(d, a, c, i, k, ridx, xm, F[c + X], e);
+      put_update(F, c, nv);
+      if (FORM != kStored) write_images<COMP>(d, a, F, i, j, k, nv);
+    }
   }
   // block sum of du^2 in a fixed order
   __shared__ double sh[512];

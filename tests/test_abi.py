@@ -9,6 +9,7 @@ import ctypes
 import os
 import re
 import shutil
+import struct
 import subprocess
 
 import pytest
@@ -74,6 +75,50 @@ def test_library_loads_and_exports_exactly_the_header():
         assert hasattr(lib, n), f"libfelgpu.so does not export {n}"
     extra = {s for s in exported(GPU_SO) if not s.startswith("_Z")} - set(names)
     assert not extra, f"exported but not declared in include/felgpu.h: {sorted(extra)}"
+
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+
+
+def kernel_private_bytes(path: str, tmp: str) -> dict[str, int]:
+    """Private (scratch) bytes a lane of every kernel in a built library, from
+    the metadata notes of the code objects it carries."""
+    blob, out = open(path, "rb").read(), {}
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    at = blob.find(magic)
+    while at >= 0:
+        entry = at + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", blob, at + len(magic))[0]):
+            off, size, n = struct.unpack_from("<QQQ", blob, entry)
+            target = blob[entry + 24:entry + 24 + n]
+            entry += 24 + n
+            if size == 0 or not target.endswith(b"gfx950"):
+                continue
+            with open(tmp, "wb") as f:
+                f.write(blob[at + off:at + off + size])
+            notes = subprocess.run([READELF, "--notes", tmp], check=True, capture_output=True,
+                                   text=True).stdout
+            for private, symbol in re.findall(
+                    r"\.private_segment_fixed_size:\s+(\d+)(?:(?!\.private_segment)[\s\S])*?"
+                    r"\.symbol:\s+(\S+)\.kd", notes):
+                out[symbol] = int(private)
+        at = blob.find(magic, at + 1)
+    return out
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="llvm-readelf not found")
+def test_colour_pair_kernels_use_no_private_memory(tmp_path):
+    """The viscous solve's kernels keep every value in registers: a spill costs
+    the hot launches time, and private memory is backed by device memory on
+    demand, which the allocation-free solve promises not to ask for."""
+    need(GPU_SO)
+    sizes = kernel_private_bytes(GPU_SO, str(tmp_path / "co"))
+    pairs = {k: v for k, v in sizes.items() if "sor_pair" in k}
+    # 3 components: pair 1/2 launches (2 coefficient forms, 3 types), pairs (those and 3 ghost
+    # forms), and the 3 ghost forms of the allocation-free solve
+    assert len(pairs) == 3 * (6 + 18 + 3)
+    spilled = {k: v for k, v in pairs.items() if v != 0}
+    assert not spilled, spilled
 
 
 def test_driver_library_exports_host_api():
