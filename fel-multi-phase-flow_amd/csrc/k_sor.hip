@@ -162,6 +162,25 @@ __device__ __forceinline__ constexpr bool shifted_w() {
   return (COMP == 0 && FORM == kLater) || (COMP == 1 && FORM != kStored);
 }
 
+// u at c-X (at c+ni where it is `shifted`) and at c.  FP32: both by one load and
+// the shifted value, which one wavefront of a row has, by another; selecting the
+// address takes two loads in all of them (pair-1/2 launches of v and w at
+// 512x128x256: 117 and 118 us, 110 and 114 so).  In FP64 the two loads are the
+// faster (v 205 us, 210 with one of 16 bytes, w 212 and 218).
+template <class T>
+__device__ __forceinline__ void get_pair(T* to, const T* u, int c, bool shifted, int ni) {
+  if constexpr (is_f32<T>) {
+    typedef float pair __attribute__((ext_vector_type(2), aligned(4)));
+    const pair p = *reinterpret_cast<const pair*>(u + (c - 1));
+    to[0] = p[0];
+    to[1] = p[1];
+    if (shifted) to[0] = u[c + ni];
+  } else {
+    to[0] = u[c + (shifted ? ni : -1)];
+    to[1] = u[c];
+  }
+}
+
 // One cell's update of component COMP (srcs/solu_sor4.f:131-175) at c = (i,j,k),
 // with the swept component's x neighbours xm = F[c-X], xp = F[c+X] supplied by
 // the caller; returns the new value (not stored) and adds du^2 to e.
@@ -169,7 +188,6 @@ template <int COMP, bool ONFLY, int FORM, class T, bool R00I>
 __device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c, int i, int k,
                                       int ridx, T xm, T xp, double& e) {
   const int X = 1, Y = d.sx, Z = d.sx * d.sy;
-  const int UX = shifted_u<COMP, FORM>() && i == 1 ? d.ni : -X;        // u(c-X)
   const int WZ = shifted_w<COMP, FORM>() && k == 1 ? d.nk * Z : -Z;    // w(c-Z)
   const int FZ = COMP == 2 && FORM == kFirst && k == 1 ? d.nk * Z : -Z;  // own (c-Z)
   T cf[15];
@@ -183,6 +201,12 @@ __device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c,
   }
   const T *un = a.un, *vn = a.vn, *wn = a.wn;
   const T h = T(0.5);
+  T u0[2], u1[2];  // u at c-X, c and at their neighbours towards the component's face
+  if (COMP != 0) {
+    const bool shifted = shifted_u<COMP, FORM>() && i == 1;
+    get_pair(u0, un, c, shifted, d.ni);
+    get_pair(u1, un, c + (COMP == 1 ? Y : Z), shifted, d.ni);
+  }
   using A = acc_t<T>;  // FP64 for FP32 storage (rounded once, at the store), else T
   T r00;
   if (R00I) {
@@ -205,15 +229,15 @@ __device__ __forceinline__ T sor_cell(const Dims& d, const SorArgs<T>& a, int c,
   } else if (COMP == 1) {
     visn = (+A(cf[4]) * A(vn[c - Z]) + A(cf[2]) * A(vn[c - Y]) + A(cf[0]) * A(xm) +
                  A(cf[1]) * A(xp) + A(cf[3]) * A(vn[c + Y]) + A(cf[5]) * A(vn[c + Z]) +
-                 A(cf[7]) * A(un[c + UX]) + A(cf[9]) * A(un[c]) + A(cf[8]) * A(un[c + UX + Y]) +
-                 A(cf[10]) * A(un[c + Y]) + A(cf[11]) * A(wn[c + WZ]) + A(cf[12]) * A(wn[c + Y + WZ]) +
+                 A(cf[7]) * A(u0[0]) + A(cf[9]) * A(u0[1]) + A(cf[8]) * A(u1[0]) +
+                 A(cf[10]) * A(u1[1]) + A(cf[11]) * A(wn[c + WZ]) + A(cf[12]) * A(wn[c + Y + WZ]) +
                  A(cf[13]) * A(wn[c]) + A(cf[14]) * A(wn[c + Y])) /
                 A(r00);
   } else {
     visn = (+A(cf[4]) * A(wn[c + FZ]) + A(cf[2]) * A(wn[c - Y]) + A(cf[0]) * A(xm) +
                  A(cf[1]) * A(xp) + A(cf[3]) * A(wn[c + Y]) + A(cf[5]) * A(wn[c + Z]) +
-                 A(cf[7]) * A(un[c + UX]) + A(cf[9]) * A(un[c]) + A(cf[8]) * A(un[c + UX + Z]) +
-                 A(cf[10]) * A(un[c + Z]) + A(cf[11]) * A(vn[c - Y]) + A(cf[13]) * A(vn[c]) +
+                 A(cf[7]) * A(u0[0]) + A(cf[9]) * A(u0[1]) + A(cf[8]) * A(u1[0]) +
+                 A(cf[10]) * A(u1[1]) + A(cf[11]) * A(vn[c - Y]) + A(cf[13]) * A(vn[c]) +
                  A(cf[12]) * A(vn[c - Y + Z]) + A(cf[14]) * A(vn[c + Z])) /
                 A(r00);
   }
