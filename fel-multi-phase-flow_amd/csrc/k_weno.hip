@@ -101,10 +101,11 @@ __device__ __forceinline__ T weno_side(T d5, T d3, T d1, T e1, T e3, T s5, T s3,
 // runs both sides, one after the other, in every wavefront whose 64 cells hold
 // both signs.  The powers of two in 2 |vel| = |vel4| / 2 go into the constant.
 //
-// FAST: without branches; for vel = 0 the m side stands for both, which is the
-// same zero while both sides are finite.  `odd` is set where they may not be:
-// the m side sets it through its weights' sum, and of the values that only the
-// p side reads, or reads twice as often, f(2) and f(3) are looked at here.
+// FAST: without branches on a lane; for vel = 0 the m side stands for both, which
+// is the same zero while both sides are finite.  `odd` is set where they may not
+// be: with a value of 1e30 or more (below it the products of eight differences,
+// scaled ones in FP32, stay in range), looked for in wavefronts that hold a zero
+// velocity, and wherever the side that is formed sets it through its weights' sum.
 template <bool FAST, class T>
 __device__ __forceinline__ T weno_up(T fm3, T fm2, T fm1, T f0, T fp1, T fp2, bool& odd) {
   const T d5 = fm2 - fm3, d3 = fm1 - fm2, d1 = f0 - fm1, e1 = fp1 - f0, e3 = fp2 - fp1;
@@ -126,10 +127,17 @@ __device__ __forceinline__ T weno5(T fm3, T fm2, T fm1, T f0, T fp1, T fp2, T fp
                                    bool& odd) {
   const T r12 = T(1.0) / T(12.0), r24 = T(0.5) * r12;
   const bool down = vel4 < T(0.0);
+  if constexpr (FAST) {
+    const bool still = !(fabs(vel4) > T(0.0));
+    if (__builtin_amdgcn_ballot_w64(still) != 0) {
+      bool small = true;
+      for (const T x : {fm3, fm2, fm1, f0, fp1, fp2, fp3}) small = small && fabs(x) < T(1.0e30);
+      odd |= still && !small;
+    }
+  }
   const T side = weno_up<FAST>(down ? fp3 : fm3, down ? fp2 : fm2, down ? fp1 : fm1, f0,
                                down ? fm1 : fp1, down ? fm2 : fp2, odd);
   if constexpr (FAST) {
-    odd |= !(fabs(vel4) > T(0.0)) && !(fabs(fp2) < T(1.0e30) && fabs(fp3) < T(1.0e30));
     return (fabs(vel4) * side) * r24;
   } else {
     if (down || vel4 > T(0.0)) return (fabs(vel4) * side) * r24;
@@ -177,7 +185,7 @@ __device__ __forceinline__ T weno_q(const T* q, T vel4, bool& odd) {
 // in FP64, 342 us in FP32 and 1.52 ms in the tangent mode; a branch per side and all components in one
 // thread took 810 us, 464 us and 2.10 ms, the one polynomial per lane alone
 // 657 us in FP64.  One
-// component per thread holds 93 registers instead of 124, which keeps 5
+// component per thread holds 90 registers instead of 124, which keeps 5
 // wavefronts on a SIMD instead of 4 and triples the threads of a small grid
 // (7.6 -> 4.6 us at 32x8x32); the three columns of one place run side by side
 // on one XCD, whose L2 they share.  Planes per thread: 633, 606 and 606 us

@@ -174,6 +174,25 @@ def test_weno_zero_and_non_finite_values(ni, nj, nk):
     assert np.array_equal(want[0][quiet], got[0][quiet], equal_nan=True)
 
 
+@pytest.mark.parametrize("flip", [False, True])
+def test_weno_zero_velocity_beside_an_overflowing_side(flip):
+    """WENO5 across a still direction where one side's weights overflow and the
+    other's, whose smoothness indicators vanish, do not: both sides count, and the
+    oracle's NaN is the library's."""
+    g = Grid(5, 16, 4, 1.0, 1.0, 1.0)
+    ramp = -2.0 ** 330 * np.maximum(0.0, 10.0 - np.arange(g.nj + 6))  # slope, then flat
+    u = np.empty(g.shape)
+    u[...] = (ramp[::-1] if flip else ramp)[None, :, None]
+
+    def args():
+        return [I(g.ni), I(g.nj), I(g.nk), D(1.0), D(1.0), D(1.0), u.copy(), g.zeros(),
+                np.ones(g.shape), g.zeros(), g.zeros(), g.zeros()]
+    want, got = run_both("cal_advu_weno5", args)
+    assert np.isnan(want[-3]).any() and (g.interior(want[-3]) == 0.0).any()
+    for a, b in zip(want[-3:], got[-3:]):
+        assert np.array_equal(a, b, equal_nan=True)
+
+
 # rows of odd and even length, the image's end inside a 16-byte run (0 to 3
 # elements over), less than one block
 @pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (5, 5, 5), (7, 5, 4), (33, 8, 10), (130, 9, 6)])
