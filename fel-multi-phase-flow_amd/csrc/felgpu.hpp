@@ -177,6 +177,10 @@ class Call {
 // for a result it has already computed.  content_version returns 0 unless
 // `host` is exactly one whole registered array of `count` doubles.
 uint64_t content_version(const void* host, size_t count);
+// The number of the registration that holds such an array: a fresh one when
+// the range is registered, or registered again, so an address that was given
+// back and registered anew is not taken for the array it held before.
+uint64_t registration(const void* host, size_t count);
 // As content_version, also for a sub-range of a registered array (a slice
 // such as phi(:,:,:,l)): a number that stays the same until a write
 // overlaps the sub-range.  0 for memory that is not registered.

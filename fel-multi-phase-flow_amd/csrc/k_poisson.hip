@@ -460,6 +460,7 @@ struct PoissonRecord {
   // from which contents of it and which table) solp_fft_tdma1_ transformed
   // the residual div - L dp instead of div
   const void* dp_host = nullptr;
+  uint64_t dp_reg = 0;  // the registration that held it (0: unregistered)
   bool warm = false;
   uint64_t dp0_ver = 0, warm_gen = 0;
   // statistics (felgpu_poisson_stats_): solves, warm starts, refinement
@@ -672,11 +673,9 @@ void tdma1_t(const Dims d, const double* div, double* phir_r, double* phir_i) {
   bool warm = false;
   if constexpr (is_f32<T>)
     warm = refine_steps() > 0 && rec.coef && rec.dp_host && rec.ni == d.ni && rec.nj == d.nj &&
-           rec.nk == d.nk && content_version(div, d.n3) != 0 &&
-           content_version(rec.dp_host, d.n3) != 0 &&
+           rec.nk == d.nk && content_version(div, d.n3) != 0 && rec.dp_reg != 0 &&
            // the last solve's array may be gone and its address another's
-           // (any FP64 array is a starting guess)
-           elem_size(rec.dp_host) == (int)sizeof(double);
+           registration(rec.dp_host, d.n3) == rec.dp_reg;
   Call c("solp_fft_tdma1_");
   const PT<T>* dv = c.in_t<PT<T>>(div, d.n3, "div");
   T* pr = c.out_t<T>(phir_r, nm, "phir_r");
@@ -728,6 +727,7 @@ void tdma3_t(const Dims d, const double* phir_r, const double* phir_i, double* d
     poisson_refine(d, ddp, warm);
     rec.warm = false;
     rec.dp_host = dp;
+    rec.dp_reg = registration(dp, d.n3);
   } else {
     fft_inverse<T>(d, pr, pi, ddp, false);
   }

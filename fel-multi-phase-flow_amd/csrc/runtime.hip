@@ -43,6 +43,7 @@ struct Range {
   // array (0: none assigned yet); kept by the entry points that write
   // exactly that box, renewed by every other write
   uint64_t shell = 0;
+  uint64_t born = 0;  // number of the registration
   // content numbers of sub-ranges (e.g. one slice phi(:,:,:,l)), assigned
   // on request and dropped by any overlapping write
   struct Sub {
@@ -555,6 +556,11 @@ void deferred_coef_flush() {
 uint64_t content_version(const void* host, size_t count) {
   const Range* g = whole_range(host, count);
   return g ? g->ver : 0;
+}
+
+uint64_t registration(const void* host, size_t count) {
+  const Range* g = whole_range(host, count);
+  return g ? g->born : 0;
 }
 
 uint64_t content_key(const void* host, size_t count) {
@@ -1182,6 +1188,7 @@ static void register_range(const void* host, const int64_t* nbytes, const int* u
     it = r.reg.emplace(p, Range{p, bytes, dev, esize, 0, nullptr, 0}).first;
   }
   note_write(it->second);
+  it->second.born = next_version();
   if (*upload)
     h2d(it->second.dev, host, n, esize);
   else

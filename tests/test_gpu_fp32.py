@@ -176,6 +176,71 @@ def test_warm_start_after_the_correction_array_is_gone():
         lib.felgpu_set_precision_(ctypes.byref(ctypes.c_int(64)))
 
 
+class Poisson32:
+    """FP32 pressure solves on registered arrays of one small grid."""
+
+    def __init__(self):
+        self.g, self.lib, self.reg = H.Grid(16, 8, 16), H.gpu(), []
+        g = self.g
+        self.modes = [np.zeros(g.ni * g.nj * g.nk) for _ in range(2)]
+        self.div, self.dp = g.zeros(), g.zeros()
+        r = np.random.default_rng(57)
+        g.interior(self.div)[...] = r.standard_normal((g.nk, g.nj, g.ni))
+        g.interior(self.div)[...] -= g.interior(self.div).mean()
+        pc = [np.zeros(g.nj + 6) for _ in range(7)]
+        self.fft = [np.zeros(g.nj + 6) for _ in range(3)]
+        H.call_gpu("cal_coef_prs", I(g.nj), D(1.0), D(1.0), D(1.0), D(1.0), *pc)
+        H.call_gpu("cal_coef_solp_fft", I(g.nj), pc[2], pc[3], *self.fft)
+
+    def __enter__(self):
+        self.lib.felgpu_set_precision_(ctypes.byref(ctypes.c_int(32)))
+        for a in (self.div, self.dp):
+            self.register(a, self.lib.felgpu_register_fp64_)
+        for a in self.modes:
+            self.register(a, self.lib.felgpu_register_)
+        return self
+
+    def register(self, a, fn):
+        fn(ctypes.c_void_p(a.ctypes.data), ctypes.byref(ctypes.c_int64(a.nbytes)),
+           ctypes.byref(ctypes.c_int(1)))
+        self.reg.append(a)
+
+    def drop(self, a):
+        self.lib.felgpu_unregister_(ctypes.c_void_p(a.ctypes.data))
+        self.reg = [x for x in self.reg if x is not a]
+
+    def solve(self):
+        g = self.g
+        head, wk = [I(g.ni), I(g.nj), I(g.nk)], [np.zeros(64) for _ in range(3)]
+        sv = np.array([g.ni, g.nj, g.nk], dtype=np.int32)
+        H.call_gpu("solp_fft_tdma1", *head, wk[0], self.div, *self.modes)
+        H.call_gpu("solp_fft_tdma2", I(0), I(1), sv, D(1.0), D(1.0), D(1.0), *self.fft, *wk,
+                   *self.modes)
+        H.call_gpu("solp_fft_tdma3", *head, wk[0], *self.modes, self.dp)
+        self.lib.felgpu_download_(ctypes.c_void_p(self.dp.ctypes.data))
+        return g.interior(self.dp).copy()
+
+    def __exit__(self, *exc):
+        for a in list(self.reg):
+            self.drop(a)
+        self.lib.felgpu_set_precision_(ctypes.byref(ctypes.c_int(64)))
+
+
+@pytest.mark.parametrize("given_back", [True, False], ids=["given back", "registered again"])
+def test_no_warm_start_from_another_registration(given_back):
+    """The last correction's address may since hold another FP64 array, or have
+    been registered again: the next solve does not start from what it holds
+    (NaN here)."""
+    with Poisson32() as p:
+        first = p.solve()
+        if given_back:
+            p.drop(p.dp)
+        p.dp[...] = np.nan
+        p.register(p.dp, p.lib.felgpu_register_fp64_)
+        second = p.solve()
+    assert np.linalg.norm(first - second) <= 1e-5 * np.linalg.norm(first)
+
+
 def test_fp32_precision_is_per_array_class():
     """Flow arrays registered with felgpu_register_ are FP32, arrays
     registered with felgpu_register_fp64_ stay FP64; a kernel asked to read
