@@ -630,6 +630,15 @@ static void poisson_refine(const Dims d, double* dp, bool warm) {
   const double tol = refine_tol();
   poisson_residual_pass(d, div, dp, rc, sums);
   double rel = residual_ratio(sums);
+  if (warm && std::isfinite(sums[0]) && !(rel <= 1.0)) {
+    // the guess was worse than none (the array may have been written since the
+    // last solve, also with NaN): dp = 0, whose residual is div
+    warm = false;
+    launch_box(Box{1, ni, 1, nj, 1, nk},
+               [=] __device__(int i, int j, int k) { dp[d.ix(i, j, k)] = 0.0; });
+    poisson_residual_pass(d, div, dp, rc, sums);
+    rel = residual_ratio(sums);
+  }
   pr.first_rel = rel;
   int it = 0;
   for (; it < steps && rel > tol; it++) {

@@ -241,6 +241,23 @@ def test_no_warm_start_from_another_registration(given_back):
     assert np.linalg.norm(first - second) <= 1e-5 * np.linalg.norm(first)
 
 
+@pytest.mark.parametrize("value", [np.nan, -np.inf, 1e30])
+def test_no_warm_start_from_a_useless_guess(value):
+    """A correction array that was overwritten since the last solve, with values
+    that no refinement brings back, does not spoil the next solve; a right-hand
+    side with a NaN still gives NaN."""
+    with Poisson32() as p:
+        first = p.solve()
+        p.dp[5, 6, 7] = value
+        p.lib.felgpu_upload_(ctypes.c_void_p(p.dp.ctypes.data))
+        second = p.solve()
+        p.div[5, 6, 7] = np.nan
+        p.lib.felgpu_upload_(ctypes.c_void_p(p.div.ctypes.data))
+        third = p.solve()
+    assert np.linalg.norm(first - second) <= 1e-5 * np.linalg.norm(first)
+    assert np.isnan(third).all()
+
+
 def test_fp32_precision_is_per_array_class():
     """Flow arrays registered with felgpu_register_ are FP32, arrays
     registered with felgpu_register_fp64_ stay FP64; a kernel asked to read
