@@ -1,6 +1,8 @@
 """The launch shapes that depend on the grid: chunk lengths of the marching
 kernels, tile edges and remainders, each against the oracle on the sizes where
 a shape changes."""
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -10,6 +12,24 @@ from felharness import D, I, Grid
 from test_gpu_kernels import check, grad, run_both
 
 pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def mode(which):
+    """The library in another of its modes: "fp32" or "tangent"."""
+    lib, c = H.gpu(), H.ctypes
+    fn, on, off = {"fp32": (lib.felgpu_set_precision_, 32, 64),
+                   "tangent": (lib.felgpu_set_tangent_, 1, 0)}[which]
+    fn(c.byref(c.c_int(on)))
+    try:
+        yield
+    finally:
+        fn(c.byref(c.c_int(off)))
+
+
+def float32(a):
+    """Values that the FP32 mode holds as they are."""
+    return a.astype(np.float32).astype(np.float64)
 
 
 # (64 x 4 blocks; one plane per thread up to 8: 4^3 and the odd grids march one
@@ -193,6 +213,86 @@ def test_weno_zero_velocity_beside_an_overflowing_side(flip):
         assert np.array_equal(a, b, equal_nan=True)
 
 
+# f(-3..2) of a stencil whose weight sum has a significand of all ones, the one
+# that a residual correction of an approximate reciprocal may leave a unit in the
+# last place low, depending on where it starts (in each the derivative's last
+# place depends on it)
+ALL_ONES = [
+    "0x1.5ac933da37283p-2 0x1.9c3cd63e28b70p-1 0x1.4b960e74a5b97p-2 -0x1.46ec1717aa384p+0 "
+    "0x1.c64089d23ece5p-1 0x1.bfed443a534cep-2",
+    "-0x1.e0d0c00daaa40p-1 0x1.a5e2ededb21eep-8 -0x1.1c496df700f17p+0 -0x1.1473ce69d79eep+0 "
+    "0x1.708b7879a8d94p+0 -0x1.ae807168d09b5p-5",
+    "-0x1.38543e84c0de1p-1 0x1.cafdb732b9abbp+0 -0x1.db1dde593df6ep-1 -0x1.6de1ffbe532ecp-2 "
+    "0x1.af8e923357f13p-1 -0x1.eb88eec79bd85p-3",
+    "-0x1.24246dde22f0bp+0 0x1.db3439dc6af07p+0 -0x1.7a3ac98873e55p-1 -0x1.63d200ecd1183p-2 "
+    "0x1.f1578407ff970p-1 0x1.ff18f61497003p-1",
+]
+
+
+@pytest.mark.parametrize("stencil", ALL_ONES, ids=range(4))
+@pytest.mark.parametrize("down", [False, True])
+def test_weno_weight_sums_of_all_ones(stencil, down):
+    """WENO5 at such a weight sum: bit for bit the oracle's."""
+    g = Grid(16, 4, 4, 1.0, 1.0, 1.0)
+    f = np.zeros(g.ni)
+    f[4:10] = [float.fromhex(x) for x in stencil.split()]
+    if down:  # the mirrored stencil, carried the other way
+        f = -f[::-1]
+    u, v = np.full(g.shape, -1.0 if down else 1.0), g.zeros()
+    v[:, :, 3:g.ni + 3] = f  # constant in y, where it carries itself
+
+    def args():
+        return [I(g.ni), I(g.nj), I(g.nk), D(1.0), D(1.0), D(1.0), u.copy(), v.copy(), g.zeros(),
+                g.zeros(), g.zeros(), g.zeros()]
+    want, got = run_both("cal_advu_weno5", args)
+    assert np.any(want[-2])
+    for a, b in zip(want[-3:], got[-3:]):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("down", [False, True])
+def test_weno_fp32_jump_beside_the_stencil(down):
+    """WENO5 in FP32 on cells whose upwind stencil ends before a jump of 2^20:
+    the weights are those of the values the stencil holds.  Small whole numbers
+    up to the jump, so the differences and indicators are exact; the bar is 16
+    roundings of the largest term |u|/6 (2 + 7 + 11) |d| of a derivative, |d| <= 6
+    the differences in a stencil."""
+    g = Grid(32, 4, 4, 1.0, 1.0, 1.0)
+    r = np.random.default_rng(20)
+    u = g.zeros()
+    u[...] = 8.0 + r.integers(-3, 4, g.ni + 6)
+    u[:, :, 20] = 2.0 ** 20
+    sign = -1.0 if down else 1.0
+    u = sign * (u[:, :, ::-1].copy() if down else u)
+
+    def args():
+        return [I(g.ni), I(g.nj), I(g.nk), D(1.0), D(1.0), D(1.0), u.copy(), g.zeros(), g.zeros(),
+                g.zeros(), g.zeros(), g.zeros()]
+    with mode("fp32"):
+        want, got = run_both("cal_advu_weno5", args)
+    clear = slice(3, 18)  # up to the cell that only misses the jump with f(2)
+    if down:
+        clear = slice(g.ni + 6 - 18, g.ni + 6 - 3)
+    a, b = (g.interior(x[-3])[..., clear.start - 3:clear.stop - 3] for x in (want, got))
+    assert np.min(np.max(np.abs(a), axis=(0, 1))) > 0.0
+    assert np.max(np.abs(a - b)) <= 16 * 2.0 ** -24 * 11.0 / 6.0 * 20.0 * 6.0
+
+
+def test_weno_fp32_non_finite_values():
+    """WENO5 in FP32 at infinities and NaN in a still flow: the cells that the
+    oracle leaves finite are the library's."""
+    g = Grid(66, 5, 18, 1 / 16, 1 / 12, 1 / 20)
+    r = np.random.default_rng(66)
+    u = np.where(r.random(g.shape) < 0.03, r.choice([np.inf, -np.inf, np.nan], g.shape), 0.0)
+    with mode("fp32"):
+        want, got = run_both("cal_advu_weno5", lambda: [
+            I(g.ni), I(g.nj), I(g.nk), D(16.0), D(12.0), D(20.0), u.copy()] + [
+                g.zeros() for _ in range(5)])
+    quiet = np.isfinite(u) & np.isfinite(np.roll(u, 1, 2)) & np.isfinite(np.roll(u, -1, 2))
+    assert np.isnan(want[-3][quiet]).any()
+    assert np.array_equal(want[-3][quiet], got[-3][quiet], equal_nan=True)
+
+
 # rows of odd and even length, the image's end inside a 16-byte run (0 to 3
 # elements over), less than one block
 @pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (5, 5, 5), (7, 5, 4), (33, 8, 10), (130, 9, 6)])
@@ -251,3 +351,79 @@ def test_streamed_differences_shapes(ni, nj, nk):
                     [x.copy() for x in f[:4]]))
     check(*run_both("calfst", lambda: [I(ni), I(nj), I(nk), D(0.81), D(8.1e-4), D(5.5)] +
                     [x.copy() for x in f[4:7]] + [rk.copy()] + [x.copy() for x in f[7:10]]))
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (5, 5, 5), (33, 8, 10), (130, 9, 6)])
+@pytest.mark.parametrize("which", ["fp32", "tangent"])
+def test_streamed_differences_in_the_other_modes(ni, nj, nk, which):
+    """The same kernels with four elements a run and with one: bit for bit the
+    oracle's in the tangent mode, in FP32 within the rounding of a scale, two
+    operations and the store, relative to each element."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    r = np.random.default_rng(ni * nj + nk)
+    f = [float32(r.standard_normal(g.shape)) for _ in range(10)]
+    rk = float32(r.standard_normal((3,) + g.shape))
+    dy = r.uniform(8.0, 16.0, nj + 6)
+    scales = [D(16.0), D(12.0), D(20.0)]
+    with mode(which):
+        both = [run_both("cal_grad_p2uvw", lambda: [I(0), I(nj), I(ni), I(nj), I(nk), scales[0],
+                                                    dy.copy(), scales[2]] +
+                         [x.copy() for x in f[:4]]),
+                run_both("cal_grad_prs", lambda: [I(ni), I(nj), I(nk)] + scales +
+                         [x.copy() for x in f[:4]]),
+                run_both("calfst", lambda: [I(ni), I(nj), I(nk), D(0.81), D(8.1e-4), D(5.5)] +
+                         [x.copy() for x in f[4:7]] + [rk.copy()] + [x.copy() for x in f[7:10]])]
+    eps = 4 * 2.0 ** -24 if which == "fp32" else 0.0
+    for want, got in both:
+        for a, b in zip(want, got):
+            if isinstance(a, np.ndarray):
+                assert np.all(np.abs(a - b) <= eps * np.abs(a))
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(4, 4, 4), (66, 7, 18), (130, 9, 6), (33, 8, 10), (8, 5, 9)])
+@pytest.mark.parametrize("which", ["fp32", "tangent"])
+@pytest.mark.parametrize("resident", [False, True], ids=["coefficients", "viscosity"])
+def test_viscous_solve_with_any_ghosts_in_the_other_modes(ni, nj, nk, which, resident):
+    """As test_viscous_solve_with_any_ghosts, interior values: bit for bit the
+    oracle's in the tangent mode; in FP32 within 16 roundings a sweep of the
+    largest velocity, 21 sweeps at most (a source read from the wrong ghost is off
+    by the size of the velocities)."""
+    g = Grid(ni, nj, nk, 1 / 16, 1 / 12, 1 / 20)
+    r = np.random.default_rng(ni * nj + nk)
+    head = [I(ni), I(nj), I(nk)]
+    rmu, rho, rhon = (float32(r.uniform(0.5, 1.0, g.shape)) for _ in range(3))
+    phi, l1, l2 = (r.uniform(0.05, 1.0, g.shape) for _ in range(3))
+    src, start = ([float32(r.standard_normal(g.shape)) for _ in range(3)] for _ in range(2))
+
+    def solve(call, coef, uvw):
+        call("cal_arith_coef_vis", *head, D(1 / g.dx), D(1 / g.dy), D(1 / g.dz), rmu, *coef)
+        call("solu_sor4", I(0), I(0), np.full(6, -1, np.int32), I(1), *head,
+             np.zeros(8, np.int32), np.zeros(8), np.zeros(8), I(1), I(0), D(0.001), rho, rhon,
+             *coef, *src, *uvw, D(0.25), D(g.dy), l1, l2, phi)
+
+    want, got = [x.copy() for x in start], [x.copy() for x in start]
+    solve(H.call_oracle, [g.zeros() for _ in range(45)], want)
+    coef = [g.zeros() for _ in range(45)]
+    with mode(which):
+        if resident:
+            lib = H.gpu()
+            flow, phase = [rmu, rho, rhon, *src, *coef, *got], [phi, l1, l2]
+            try:
+                for a in flow + phase:
+                    fn = lib.felgpu_register_ if any(a is x for x in flow) else lib.felgpu_register_fp64_
+                    fn(H.ctypes.c_void_p(a.ctypes.data), H.ctypes.byref(H.ctypes.c_int64(a.nbytes)),
+                       H.ctypes.byref(H.ctypes.c_int(1)))
+                solve(H.call_gpu, coef, got)
+                for a in got:
+                    lib.felgpu_download_(H.ctypes.c_void_p(a.ctypes.data))
+            finally:
+                for a in flow + phase:
+                    lib.felgpu_unregister_(H.ctypes.c_void_p(a.ctypes.data))
+        else:
+            solve(H.call_gpu, coef, got)
+    for a, b in zip(want, got):
+        if which == "tangent":
+            assert np.array_equal(a, b)
+        else:
+            a, b = g.interior(a), g.interior(b)
+            assert np.max(np.abs(a - b)) <= 21 * 16 * 2.0 ** -24 * np.max(np.abs(a))
