@@ -350,7 +350,7 @@ bool chain_deferral_enabled();
 void deferred_chain_flush();
 void deferred_chain_check(const void* host, bool write);
 
-// Pinned host scratch for small device->host read-backs (reductions).
+// Waits for the library's stream.
 void sync();
 
 // Device scratch reused across calls (grows, never shrinks).
@@ -627,7 +627,7 @@ __global__ void __launch_bounds__(256) sum_stage2(int nb, const A* part, double*
   }
 }
 
-// Runs both stages; `out` is device memory.  f(i, j, k, A* v) gives the NV
+// Runs both stages; `out` is device memory, or pinned host memory.  f(i, j, k, A* v) gives the NV
 // addends of cell (i,j,k); g(const A* totals, double* out) stores results.
 template <int NV, class A = double, class F, class G>
 inline void interior_reduce(const Dims& d, F f, G g, double* out) {

@@ -804,8 +804,10 @@ SorResult solu_sor4_t(const Dims d, double dt, const double* rho, const double* 
 
 // ---------------------------------------------------------------------------
 // Allocation-free solve (felgpu_solu_sor4_noalloc_): its work memory -- the
-// residual partials, the residual sum and the slip-wall coefficients -- lives
-// in this static device array instead of library-allocated buffers.  Each
+// residual partials and the slip-wall coefficients -- lives in this static
+// device array instead of library-allocated buffers; the residual sum is
+// written to the pinned host memory that the library's initialisation
+// allocates, the slot that solu_sor4_ uses.  Each
 // device holds its own copy at its own address, found once per device with
 // hipGetSymbolAddress (fel::sor_noalloc_setup, called from the library's
 // initialisation) and used through that address only: the array's name in

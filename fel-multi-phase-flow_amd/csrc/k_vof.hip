@@ -3,8 +3,10 @@
 //
 // Reference: srcs/cal_grad_p2a.f, srcs/solphi_mthinc1.f (+ mthinc_x.h,
 // mthinc_tanh.h), srcs/solphi_mthinc2.f, srcs/solphi_mthinc3.f,
-// srcs/summation.f.  All FP64, expressions evaluated in the reference's
-// order (the library is compiled without contraction).
+// srcs/summation.f.  Expressions are evaluated in the reference's order (the
+// library is compiled without contraction), except in the interface cells of the
+// MTHINC fluxes: the eight Gauss points are added pairwise, and the sigmoid's
+// derivative is formed from the sigmoid.
 #include <cmath>
 
 #include <cstdlib>
@@ -100,8 +102,10 @@ static MthincConst mthinc_const(double dxinv, double dyinv, double dzinv, double
 // iterations and Gauss sums of the listed cells.  One launch of one thread per
 // cell kept a wave busy with ten serial Newton steps of eight Gauss points
 // wherever a single lane met the interface, and could not march in k.
-// Measured (one droplet, FP64): 571 -> 371 + 22 us at 512x256x128, 110 -> 14
-// us at 32x8x32.
+// Measured (one droplet, FP64): 571-593 -> 371 + 22 us in a flow that moves
+// everywhere and 322 + 23 us in the droplet impact's, at 512x128x256; 110 -> 14
+// us at 32x8x32.  In a host emulation the pairwise sums' fluxes are off by
+// 1.06e-16 (relative 2-norm) from extended precision, serial sums' by 1.36e-16.
 //
 // T: element type of the gradients, the velocities and of the MTHINC
 // arithmetic (double, or float in the FP32 mode); the fluxes are stored in
@@ -318,7 +322,8 @@ void mthinc_update(const Dims d, double dxinv, double dyinv, double dzinv, doubl
 // thread per (i,j) column, marching over up to kMassChunk planes: the 8-point
 // averages of the gradients take their k-1 plane from the values the column
 // loaded for the previous plane, so each plane of phix, phiy, phiz is
-// fetched once per column.  The sums are vavg8's, in its order.
+// fetched once per column.  The sums keep the reference's order: plane k-1, then
+// plane k, each from (i-1,j-1) to (i,j).
 // (measured at 512x256x128 in FP64: 177 us with 8 planes, 183 with 2, 176
 // with 4, 180 with 16)
 constexpr int kMassChunk = 8;

@@ -20,7 +20,9 @@ namespace fel {
 // that brings their largest magnitude to [1, 2): the weights are homogeneous
 // of degree 0 in that scale, so the scaling changes nothing but keeps the
 // degree-8 products of the smoothness indicators inside the FP32 range; the
-// stencil derivatives use the unscaled differences.
+// stencil derivatives use the unscaled differences.  The scale is that of the
+// five differences the upwind side reads: a sixth, much larger one beside them
+// would push the weight sums under their floor.
 // 1/x for the weights: IEEE division in FP64 (and the tangent mode); in the
 // FP32 mode the hardware reciprocal (v_rcp_f32, 1 ulp), whose rounding is
 // far below the FP32 mode's accuracy bar and which replaces a ten-instruction
@@ -29,7 +31,10 @@ namespace fel {
 // FAST (FP64): the quotient by Newton's iteration from the hardware reciprocal
 // with the final residual correction (Markstein), which is the correctly
 // rounded 1/x where no step leaves the normal range; the weight sums are at
-// least 1e-80, and one of 1e300 or more (or NaN) sets `odd`.
+// least 1e-80, and one of 1e300 or more (or NaN) sets `odd`.  (The one divisor
+// for which the iteration may end a unit low, a significand of all ones, does
+// not: gfx950's approximation of it is the rounded quotient already, at every
+// exponent, and the steps keep it.)
 template <bool FAST, class T>
 __device__ __forceinline__ T weight_rcp(T x, bool& odd) {
   if constexpr (is_f32<T>) {
@@ -45,12 +50,6 @@ __device__ __forceinline__ T weight_rcp(T x, bool& odd) {
   }
 }
 
-// One upwind-biased side of srcs/weno5.h: w1*df1 + w2*df2 + w3*df3 of the
-// side whose differences are (d5, d3, d1, e1, e3) -- the m side (dfm5,
-// dfm3, dfm1, dfp1, dfp3), the p side mirrored (dfp5, dfp3, dfp1, dfm1,
-// dfm3) -- with the candidate derivatives from those differences and the
-// smoothness indicators from their scaled copies (s5, s3, s1, t1, t3);
-// expressions in the reference's order.
 // p x + y with p a power of two, where the reference rounds p x and then the
 // sum: p x is exact, so one fused operation gives the same bits.
 template <class T>
@@ -59,6 +58,12 @@ __device__ __forceinline__ T pow2_fma(double p, T x, T y) {
   else return x * T(p) + y;
 }
 
+// One upwind-biased side of srcs/weno5.h: w1*df1 + w2*df2 + w3*df3 of the
+// side whose differences are (d5, d3, d1, e1, e3) -- the m side (dfm5,
+// dfm3, dfm1, dfp1, dfp3), the p side mirrored (dfp5, dfp3, dfp1, dfm1,
+// dfm3) -- with the candidate derivatives from those differences and the
+// smoothness indicators from their scaled copies (s5, s3, s1, t1, t3);
+// expressions in the reference's order.
 template <bool FAST, class T>
 __device__ __forceinline__ T weno_side(T d5, T d3, T d1, T e1, T e3, T s5, T s3, T s1, T t1,
                                        T t3, bool& odd) {
@@ -181,15 +186,16 @@ __device__ __forceinline__ T weno_q(const T* q, T vel4, bool& odd) {
 // are loaded from the same plane, which the block's other lanes share in cache.
 //
 // Bound by the FP64 units: about 95 operations a derivative, issued in 75% of
-// the cycles.  Measured at 512x128x256 with velocities of both signs: 606 us
-// in FP64, 342 us in FP32 and 1.52 ms in the tangent mode; a branch per side and all components in one
-// thread took 810 us, 464 us and 2.10 ms, the one polynomial per lane alone
-// 657 us in FP64.  One
-// component per thread holds 90 registers instead of 124, which keeps 5
-// wavefronts on a SIMD instead of 4 and triples the threads of a small grid
-// (7.6 -> 4.6 us at 32x8x32); the three columns of one place run side by side
-// on one XCD, whose L2 they share.  Planes per thread: 633, 606 and 606 us
-// with 4, 8 and 16.
+// the cycles.  Measured at 512x128x256 with velocities of both signs everywhere:
+// 606-625 us in FP64, 331-342 us in FP32 and 1.52 ms in the tangent mode; a
+// branch per side and all components in one thread took 810 us, 464 us and
+// 2.10 ms, the one polynomial per lane alone 657 us in FP64.  In a flow whose
+// wavefronts mostly hold one sign (the droplet impact) the branch cost little:
+// 636 -> 612 us.  One component per thread holds 90 registers instead of 124,
+// which keeps 5 wavefronts on a SIMD instead of 4 and triples the threads of a
+// small grid (7.6 -> 4.6 us at 32x8x32); the three columns of one place run side
+// by side on one XCD, whose L2 they share.  Planes per thread: 633, 606 and 606
+// us with 4, 8 and 16.
 constexpr int kWenoK = 8;
 
 template <int COMP, class T>

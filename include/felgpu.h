@@ -314,7 +314,10 @@ void felgpu_sor_last_(int *lp, double *ratio);
  * formed in the sweep kernels) lives in a static 16 MiB device array per
  * GPU, located once per device at the library's initialisation: the call
  * allocates nothing.  Limit: grids whose work memory exceeds 16 MiB
- * (8 (12 nb + 257) + 32 (ni+6)(nk+6) bytes, nb the blocks of one launch;
+ * (8 (12 nb + 256) rounded up to a multiple of 256, and 32 (ni+6)(nk+6)
+ * bytes, nb the blocks of the larger launch: ceil(ni/128) ceil(nj/8) nk of a
+ * colour pair, ceil(nj/2) nk of pairs 1 and 2 together where ni and nk are
+ * even and ni is 1024 at most;
  * 5.9 MB at 512x128x256, 14.9 MB at 512x256x512) are refused.  Calls that
  * overlap on one GPU race on that array.  *lp, *ratio: as felgpu_sor_last_.
  * Returns 0; 1 when the grid needs more work memory than the array holds;
